@@ -281,211 +281,174 @@ struct LowerAcc {
 // ---- D_K --------------------------------------------------------------------
 // The task takes the 64x64 tile S (lower part; the part above the diagonal is
 // never read) in LDS as xs[col][row], writes D to piv and Linv = L^{-1} (zeros
-// above the diagonal) to lout, and overwrites xs.  L_KK itself is read by
-// neither the panels and updates nor the solves and is not stored.  FP32
+// above the diagonal) to lout, and overwrites xs and ys.  L_KK itself is read
+// by neither the panels and updates nor the solves and is not stored.  FP32
 // tiles go through the FP64 task (below).
+//
+// FP64, blocked by 16: [S | I] is eliminated by block columns k = 0..3.
+//  - Wavefront 0 runs the 16 pivot steps of block column k in its registers.
+//    Each of its four 16-lane rows holds the 16x16 diagonal block (lane j:
+//    row j, a[c] = A_jc) and one 16x16 block of right-hand sides of the same
+//    elimination (lane j: x[c], c = 0..15).  Row g carries block (k + g) mod 4:
+//    the identity for g = 0, which becomes Linv_kk; A_ik^T for a block row i
+//    below, which becomes (L_ik D_k)^T; and for a block column j to the left
+//    B_kj = -sum_{m<k} L_km Linv_mj, which becomes Linv_kj.  So the four rows
+//    always have one block each and Linv is complete with the last pivot.
+//    Step c needs a[c] alone: the pivot and the factor of row i are its lanes
+//    c and i, which reach the whole 16-lane row as DPP operands (row_newbcast)
+//    of the FP64 multiply-adds.  The next pivot is formed first and its
+//    reciprocal while the rest of the step issues.
+//  - After a barrier wavefronts 0..3 update what block column k + 1 needs
+//    (FP64 MFMA 16x16x4, four steps per 16x16 block); the blocks of the later
+//    columns follow on the other wavefronts during the next pivot steps,
+//    except wavefront 4, which shares a SIMD with wavefront 0.
+// xs column 16k + c receives -L_ik in rows 16i.. (and -x/d elsewhere), ys row
+// 16k + c the right-hand sides: Linv row by row up to the diagonal and L D
+// beyond it.  Multipliers are l = a / d as a * (1/d), with the reciprocal's
+// correction applied to the product.
+// What bounds it is the chain of 64 pivots: reciprocal (28 cycles), its
+// correction, multiplier and next pivot (8 cycles an FP64 operation), and 5.5
+// cycles for each of a step's up to 30 multiply-adds.  One tile on an idle GPU
+// takes 7.3 us; with the columns broadcast through LDS, the blocks of Linv
+// formed beside and after the pivots, it took 12.1 us (pivots then came at 370
+// cycles each, now at about 190).
 template <class R> struct DiagScratch;
-template <> struct DiagScratch<double> { double tsc[5][256]; double ub[16]; };
-// FP64: blocked by 16.  For each column block k:
-//  - wavefront 0 factorizes the 64x16 panel (rows 16k..63, lane = row):
-//    16 pivot steps, each broadcasting column c of the block through LDS; the
-//    pivot and the next step's critical entry travel by readlane, and the
-//    reciprocal of the next pivot is formed while the rest of the step's
-//    updates are issued.  The block lanes also form column p of Linv_kk by
-//    the same elimination applied to the identity.  Multipliers are
-//    l = a * (1/d) with the reciprocal refined by two Newton steps.
-//  - the other wavefronts meanwhile form the off-diagonal blocks of Linv
-//    that are ready, Linv_ij = -Linv_ii sum_{k=j}^{i-1} L_ik Linv_kj, as
-//    16x16x16 FP64 MFMA products, avoiding wavefront 4 (which shares a SIMD
-//    with wavefront 0);
-//  - after a barrier, up to six wavefronts update the trailing blocks
-//    A_ij -= L_ik D_k L_jk^T (16x16x16 FP64 MFMA).
-// Linv is kept in ys column-major with the row index swizzled by the column
-// (ysw), which makes both row and column accesses free of bank conflicts.
+template <> struct DiagScratch<double> { double dg[16][16]; };   // a[c] of every lane when column c's pivot is taken
 
-__device__ __forceinline__ int ysw(int col, int row) { return col * T + (row ^ (col & 15)); }
+// ys index of row c, column r: the columns of a row are permuted so that both
+// rows and columns are read without bank conflicts
+__device__ __forceinline__ int ysw(int c, int r) { return c * T + (r ^ ((c & 3) << 4 | (c >> 2 & 15))); }
 
-__device__ __forceinline__ double lane_value(double x, int lane) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
-    const unsigned lo = __builtin_amdgcn_readlane(unsigned(u), lane);
-    const unsigned hi = __builtin_amdgcn_readlane(unsigned(u >> 32), lane);
-    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+// The pivot steps' operations are volatile so that they issue in the order
+// written: a DPP operand must not have been written by either of the two
+// instructions in front.
+template <int I> __device__ __forceinline__ void fmac_lane(double& acc, double ac, double m) {   // acc += ac(lane I) m
+    __asm__ volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                     : "+v"(acc) : "v"(ac), "v"(m), "n"(I));
+}
+template <int I, int E>
+__device__ __forceinline__ void fmac_lanes(double* a, double* x, double ac, double m, double l) {   // i = I .. E-1
+    if constexpr (I < E && I < 16) {
+        fmac_lane<I>(a[I], ac, m);
+        fmac_lane<I>(x[I], ac, l);
+        fmac_lanes<I + 1, E>(a, x, ac, m, l);
+    }
+}
+template <int C> __device__ __forceinline__ double row_lane(double v) {   // v of lane C
+    double r;
+    __asm__ volatile("v_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(v), "n"(C));
+    return r;
 }
 
-__device__ __forceinline__ double recip(double d) {
-    double r = __builtin_amdgcn_rcp(d);
-    double e = __builtin_fma(-d, r, 1.0);
-    r = __builtin_fma(r, e, r);
-    e = __builtin_fma(-d, r, 1.0);
-    return __builtin_fma(r, e, r);
-}
-
-// D[m][n] = sum_t A(m, t) B(t, n) over 16x16 blocks on one wavefront (FP64
-// MFMA 16x16x4: lane l supplies A(l%16, t) and B(t, l%16), t = t0 + l/16);
-// element e of lane l is D[l/16 + 4e][l%16].
-template <class FA, class FB>
-__device__ __forceinline__ d4 mm16(FA A, FB B, d4 acc) {
-    const int l = threadIdx.x & 63, rr = l & 15, lg = l >> 4;
-#pragma unroll
-    for (int t0 = 0; t0 < 16; t0 += 4) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A(rr, t0 + lg), B(t0 + lg, rr), acc, 0, 0, 0);
-    return acc;
+// Steps C .. 15: r is 1/d of pivot d = a[C] (lane C) to a relative error e
+// below 2^-23 and e2 = e + e^2, so that 1/d is r + r e2.  xs, dg: this lane's
+// entry of row 0 of the block and of the pivot columns; off: its byte offset
+// in a row of ys before the row's permutation.
+template <int C>
+__device__ __forceinline__ void pivot_steps(double* a, double* x, double r, double q, double e2, double* xs, char* ysb,
+                                            int off, double* dg) {
+    const double ac = a[C], xc = x[C];
+    double m, l, rd;
+    __asm__ volatile("v_fma_f64 %0, -%1, %2, -%1" : "=v"(m) : "v"(q), "v"(e2));          // -a[C] / d
+    __asm__ volatile("v_fma_f64 %0, -%1, %2, -%1" : "=v"(rd) : "v"(r), "v"(e2));         // -1 / d
+    if constexpr (C < 15) fmac_lane<C + 1>(a[C + 1], ac, m);
+    __asm__ volatile("v_mul_f64 %0, %1, %2" : "=v"(l) : "v"(xc), "v"(rd));               // -x[C] / d
+    double rn = 0.0, en = 0.0, qn = 0.0, e2n = 0.0;
+    if constexpr (C < 15) {
+        if constexpr (C < 14) fmac_lane<C + 2>(a[C + 2], ac, m);
+        else __asm__ volatile("s_nop 0");
+        const double dn = row_lane<C + 1>(a[C + 1]);
+        fmac_lane<C + 1>(x[C + 1], ac, l);
+        __asm__ volatile("v_rcp_f64 %0, %1" : "=v"(rn) : "v"(dn));
+        if constexpr (C < 14) fmac_lane<C + 2>(x[C + 2], ac, l);
+        fmac_lanes<C + 3, C + 5>(a, x, ac, m, l);
+        if constexpr (C > 12) __asm__ volatile("s_nop 0");
+        __asm__ volatile("v_fma_f64 %0, -%1, %2, 1.0" : "=v"(en) : "v"(dn), "v"(rn));
+        __asm__ volatile("v_mul_f64 %0, %1, %2" : "=v"(qn) : "v"(a[C + 1]), "v"(rn));
+        fmac_lanes<C + 5, C + 6>(a, x, ac, m, l);
+        __asm__ volatile("v_fma_f64 %0, %1, %1, %1" : "=v"(e2n) : "v"(en));
+        fmac_lanes<C + 6, 16>(a, x, ac, m, l);
+    }
+    xs[C * T] = l;
+    *reinterpret_cast<double*>(ysb + C * T * 8 + (off ^ ((C & 3) << 7 | C >> 2 << 3))) = xc;
+    dg[C * 16] = ac;
+    if constexpr (C < 15) pivot_steps<C + 1>(a, x, rn, qn, e2n, xs, ysb, off, dg);
 }
 
 struct NoHook {
     __device__ void operator()() const {}
 };
 
-// tail_hook runs once the pivot steps are done (every thread), where few
-// registers are live: a caller issues loads there that it consumes after the
-// task.
-template <class Hook = NoHook, class O = double>
+// tail_hook runs once before the last block column's pivot steps (every
+// thread): a caller issues loads there that it consumes after the task.  CO:
+// D and Linv are stored coherently, for readers in the same launch.
+template <bool CO = false, class Hook = NoHook, class O = double>
 __device__ __forceinline__ void diag_task(double (*xs)[T], double* ys, double* dd, DiagScratch<double>& sm,
                                           O* __restrict__ lout, double* __restrict__ piv, long Kt,
                                           double* lds_out = nullptr, Hook tail_hook = Hook()) {
     const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, rr = l & 15, lg = l >> 4;
-    double(*tsc)[256] = sm.tsc;
-    // operand views: L_ik (rows r, cols t), Linv_ij as (t, c) and as (r, t), T slot s as (t, c)
-    auto Lb = [&](int i, int k) { return [&, i, k](int r, int t) { return xs[16 * k + t][16 * i + r]; }; };
-    auto Vb = [&](int i, int j) { return [&, i, j](int t, int c) { return ys[ysw(16 * j + c, 16 * i + t)]; }; };
-    auto Vr = [&](int i, int j) { return [&, i, j](int r, int t) { return ys[ysw(16 * j + t, 16 * i + r)]; }; };
-    auto Tb = [&](int s) { return [&, s](int t, int c) { return tsc[s][t * 16 + c]; }; };
-    auto getT = [&](int s) {
-        d4 acc;
+    // block (q, p) of the elimination after block column m: A_qp (q >= p > m)
+    // or B_pq (q <= m; its first contribution when q = m)
+    // (the sixteen products are summed before they meet the entry, which
+    // costs one rounding at its magnitude instead of four)
+    auto trail = [&](int m, int p, int q) {
+        d4 old = {0.0, 0.0, 0.0, 0.0}, acc = {0.0, 0.0, 0.0, 0.0};
+        if (q != m) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] = tsc[s][(lg + 4 * e) * 16 + rr];
-        return acc;
-    };
-    auto putT = [&](int s, d4 acc) {
+            for (int e = 0; e < 4; ++e) old[e] = xs[16 * p + lg + 4 * e][16 * q + rr];
+        }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) tsc[s][(lg + 4 * e) * 16 + rr] = acc[e];
-        __builtin_amdgcn_wave_barrier();
-    };
-    auto putV = [&](int i, int j, d4 acc) {   // Linv_ij = -acc
+        for (int t0 = 0; t0 < 16; t0 += 4) {
+            const int t = 16 * m + t0 + lg;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(xs[t][16 * p + rr], ys[ysw(t, 16 * q + rr)], acc, 0, 0, 0);
+        }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ys[ysw(16 * j + rr, 16 * i + lg + 4 * e)] = -acc[e];
-        __builtin_amdgcn_wave_barrier();
+        for (int e = 0; e < 4; ++e) xs[16 * p + lg + 4 * e][16 * q + rr] = old[e] + acc[e];
     };
-    const d4 z = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll 1
     for (int k = 0; k < 4; ++k) {
+        if (k == 3) tail_hook();
         if (wv == 0) {
-            const int r = l, base = 16 * k, p = r - base;
-            double v[16], bcol[16];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                v[q] = xs[base + q][r];
-                bcol[q] = (q == p) ? 1.0 : 0.0;
-            }
-            if (p >= 0 && p < 16) sm.ub[p] = v[0];
-            __builtin_amdgcn_wave_barrier();
-            double d = lane_value(v[0], base);
-            double rd = recip(d);
-            double dr = 0.0;
-            double U[16];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) U[q] = sm.ub[q];
+            const int base = 16 * k, row = 16 * ((k + lg) & 3) + rr;
+            double a[16], x[16];
 #pragma unroll
             for (int c = 0; c < 16; ++c) {
-                int po = p;
-                __asm__ volatile("" : "+v"(po));   // keeps the per-step lane tests in the step
-                const bool below = po > c;
-                dr = (po == c) ? d : dr;
-                const double le = below ? v[c] * rd : 0.0;
-                const double fb = below ? 0.0 : bcol[c] * rd;
-                double dn = 0.0, rdn = 0.0, un = 0.0;
-                if (c + 1 < 16) {
-                    v[c + 1] = __builtin_fma(-le, U[c + 1], v[c + 1]);
-                    __builtin_amdgcn_wave_barrier();
-                    if (po >= 0 && po < 16) sm.ub[po] = v[c + 1];
-                    __builtin_amdgcn_wave_barrier();
-                    dn = lane_value(v[c + 1], base + c + 1);
-                    if (c + 2 < 16) un = lane_value(v[c + 1], base + c + 2);
-                    rdn = recip(dn);
-                }
-#pragma unroll
-                for (int q = c + 2; q < 16; ++q) v[q] = __builtin_fma(-le, U[q], v[q]);
-#pragma unroll
-                for (int q = c + 1; q < 16; ++q) bcol[q] = __builtin_fma(-fb, U[q], bcol[q]);
-                v[c] = below ? le : v[c];
-                if (c + 1 < 16) {
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) U[q] = (q == c + 2) ? un : sm.ub[q];
-                    d = dn;
-                    rd = rdn;
-                }
-                // keep every update in its own step (no deferred chains)
-#pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    __asm__ volatile("" : "+v"(v[q]));
-                    __asm__ volatile("" : "+v"(bcol[q]));
-                }
+                a[c] = xs[base + c][base + rr];
+                x[c] = xs[base + c][row];
             }
-            if (p >= 0) {
 #pragma unroll
-                for (int q = 0; q < 16; ++q) xs[base + q][r] = v[q];
-            }
-            if (p >= 0 && p < 16) {
-                dd[r] = dr;
-                piv[Kt * T + r] = dr;
-#pragma unroll
-                for (int q = 0; q < 16; ++q) ys[ysw(base + p, base + q)] = (q >= p) ? bcol[q] : 0.0;
+            for (int c = 0; c < 16; ++c) x[c] = (lg == 0) ? (c == rr ? 1.0 : 0.0) : x[c];
+            __asm__ volatile("s_nop 1" : "+v"(a[0]));
+            const double d = row_lane<0>(a[0]), r = __builtin_amdgcn_rcp(d), e = __builtin_fma(-d, r, 1.0);
+            pivot_steps<0>(a, x, r, a[0] * r, __builtin_fma(e, e, e), &xs[base][row],
+                           reinterpret_cast<char*>(ys + base * T), (row ^ 4 * k) * 8, &sm.dg[0][rr]);
+            if (l < 16) {
+                const double dl = sm.dg[l][l];
+                dd[base + l] = dl;
+                cst<CO>(&piv[Kt * T + base + l], dl);
             }
         } else if (k == 1) {
-            if (wv == 1) putT(0, mm16(Lb(1, 0), Vb(0, 0), z));                      // T_10
+            // after block column 0: blocks of the columns 2 and 3
+            if (wv == 1) trail(0, 2, 0);
+            else if (wv == 2) trail(0, 2, 2);
+            else if (wv == 3) trail(0, 2, 3);
+            else if (wv == 5) trail(0, 3, 0);
+            else if (wv == 6) trail(0, 3, 3);
         } else if (k == 2) {
-            if (wv == 1) {
-                putV(1, 0, mm16(Vr(1, 1), Tb(0), z));                                // Linv_10
-                putT(1, mm16(Lb(2, 1), Vb(1, 0), mm16(Lb(2, 0), Vb(0, 0), z)));      // T_20
-            } else if (wv == 2) {
-                putT(2, mm16(Lb(2, 1), Vb(1, 1), z));                                // T_21
-            } else if (wv == 3) {
-                putT(3, mm16(Lb(3, 0), Vb(0, 0), z));                                // T_30, first term
-            } else if (wv == 5) {
-                putT(4, mm16(Lb(3, 1), Vb(1, 1), z));                                // T_31, first term
-            }
-        } else if (k == 3) {
-            if (wv == 1) putV(2, 0, mm16(Vr(2, 2), Tb(1), z));                       // Linv_20
-            else if (wv == 2) putV(2, 1, mm16(Vr(2, 2), Tb(2), z));                  // Linv_21
-            else if (wv == 3) putT(3, mm16(Lb(3, 1), Vb(1, 0), getT(3)));            // T_30, second term
-            else if (wv == 5) putT(0, mm16(Lb(3, 2), Vb(2, 2), z));                  // T_32
+            if (wv == 1) trail(1, 3, 0);
+            else if (wv == 2) trail(1, 3, 1);
+            else if (wv == 3) trail(1, 3, 3);
         }
         __syncthreads();
-        if (k == 3) break;
-        // trailing update of the blocks k < j <= i <= 3, one per wavefront
-        {
-            const int nb = 3 - k;
-            int pp = wv, i = -1, j = -1;
-            for (int a = 0; a < nb && i < 0; ++a)
-                for (int b = 0; b <= a; ++b) {
-                    if (pp == 0) { i = k + 1 + a; j = k + 1 + b; break; }
-                    --pp;
-                }
-            if (i >= 0) {
-                // D[m = c][n = r] = sum_t L_jk[c][t] (L_ik[r][t] d_t)
-                const d4 acc = mm16([&](int c, int t) { return xs[16 * k + t][16 * j + c]; },
-                                    [&](int t, int r) { return xs[16 * k + t][16 * i + r] * dd[16 * k + t]; }, z);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) xs[16 * j + lg + 4 * e][16 * i + rr] -= acc[e];
-            }
+        if (k < 3) {
+            if (wv < 4) trail(k, k + 1, wv);
+            __syncthreads();
         }
-        __syncthreads();
     }
-    tail_hook();
-    // the last row of blocks: T_3j completed, Linv_3j = -Linv_33 T_3j
-    if (wv == 0) {
-        putT(1, mm16(Lb(3, 2), Vb(2, 0), getT(3)));
-        putV(3, 0, mm16(Vr(3, 3), Tb(1), z));
-    } else if (wv == 1) {
-        putT(2, mm16(Lb(3, 2), Vb(2, 1), getT(4)));
-        putV(3, 1, mm16(Vr(3, 3), Tb(2), z));
-    } else if (wv == 2) {
-        putV(3, 2, mm16(Vr(3, 3), Tb(0), z));
-    }
-    __syncthreads();
     for (int idx = threadIdx.x; idx < TT; idx += NTH) {
         const int col = idx / T, row = idx % T;
-        const double v = (row >= col) ? ys[ysw(col, row)] : 0.0;
-        lout[idx] = O(v);
+        const double v = (row >= col) ? ys[ysw(row, col)] : 0.0;
+        cst<CO>(&lout[idx], O(v));
         if (lds_out) lds_out[idx] = v;
     }
 }
@@ -496,11 +459,12 @@ __device__ __forceinline__ void diag_task(double (*xs)[T], double* ys, double* d
 // barrier per pivot made the FP32 column launch slower than the FP64 one.
 template <> struct DiagScratch<float> { double xd[T][T]; double yd[TT]; DiagScratch<double> in; };
 
+template <bool CO = false>
 __device__ __forceinline__ void diag_task(float (*xs)[T], float* /*ys*/, double* dd, DiagScratch<float>& sm,
                                           float* __restrict__ lout, double* __restrict__ piv, long Kt) {
     for (int idx = threadIdx.x; idx < TT; idx += NTH) (&sm.xd[0][0])[idx] = double((&xs[0][0])[idx]);
     __syncthreads();
-    diag_task(sm.xd, sm.yd, dd, sm.in, lout, piv, Kt);
+    diag_task<CO>(sm.xd, sm.yd, dd, sm.in, lout, piv, Kt);
 }
 
 // ---- staging ----------------------------------------------------------------
