@@ -9,16 +9,14 @@
 namespace cb {
 
 // Kernel families of the band solver whose launches can be timed with HIP
-// events: KT_COLUMN is the fused per-column factorization launch; KT_DIAG,
+// events: KT_COLUMN is the fused factorization, per tile column; KT_DIAG,
 // KT_PANEL and KT_UPDATE are the launches of the split schedule.
 // KT_PREP times the launch that forms the sweeps' chain matrices after a
 // factorization.
 enum { KT_COLUMN = 0, KT_DIAG = 1, KT_PANEL = 2, KT_UPDATE = 3, KT_FWD = 4, KT_BWD = 5, KT_PREP = 6, KT_N = 7 };
 
 // Launches of a selected family are bracketed by two events.  The fused
-// factorization's nt launches are bracketed as one span (its launch period:
-// kernel time plus the gaps between the launches, without event overhead per
-// launch); of the split schedule's launches only every `every`-th is timed;
+// factorization is one launch and counts as its nt tile columns; of the split schedule's launches only every `every`-th is timed;
 // the sweeps are always timed.  launches counts every launch issued and ms is
 // the timed total scaled to all of them, so ms / launches is the average
 // launch duration.
@@ -82,10 +80,9 @@ struct BandLDLT {
     double* xw = nullptr;    // work vectors (padded)
     double* yw = nullptr;
     int* flag = nullptr;       // error bits: 1 a wait bound hit, 2 an entry outside the band
-    int* pflags = nullptr;     // panel completion epochs of the fused factorization launch
-    int cepoch = 0;            // epoch of the last fused launch
-    // factorization schedule: one fused launch per tile column (default), or
-    // separate diag/panel/update launches
+    int* prog = nullptr;       // progress counters of the fused factorization launch
+    // factorization schedule: one launch for all columns (default), or
+    // separate diag/panel/update launches per column
     bool split = false;
     // the tangent comes from d.K32 (the FP32 joint blocks) instead of d.K
     bool src32 = false;

@@ -66,19 +66,15 @@ __global__ void k_band_pad(R* __restrict__ tiles, long n, long nt, int w) {
 //   P_{I,K}      L_IK = A_IK Linv_K^T D_K^{-1},            K < I <= K+m
 //   U_{I,J,K}    A_IJ -= (L_IK D_K) L_JK^T,               K < J <= I <= K+m
 // (m = min(w, nt-1-K)).  Two schedules run the same tile arithmetic:
-//  - fused (default): one launch per column, k_band_column(K) for K = -1 ..
-//    nt-2.  Workgroup 0 runs the critical chain P_{K+1,K} -> U_{K+1,K+1,K} ->
-//    D_{K+1} entirely in its LDS; workgroups 1..m-1 run the other panels and
-//    the rest run the updates, each waiting on the flags of the two panels it
-//    reads.  A workgroup only waits on workgroups with a lower index, which
-//    were dispatched before it, so every wait ends; waits are bounded anyway.
+//  - fused (default): one launch, k_band_factor, whose workgroups hand tiles
+//    to each other through progress counters;
 //  - split: three launches per column (diag, panels, updates), for timing
 //    the tile tasks one by one.
-// Tiles handed between workgroups of one launch (the panels L_IK) are stored
-// and loaded with system-scope coherent accesses (written through to memory,
-// read past the XCD caches): a producer waits for its stores to complete
-// (vmcnt 0) before the flag store, a consumer reads the data after it has
-// seen the flag.  Everything else crosses a launch boundary.
+// Tiles handed between workgroups of one launch are stored and loaded with
+// system-scope coherent accesses (written through to memory, read past the
+// XCD caches): a producer waits for its stores to complete (vmcnt 0) before
+// it raises the counter, a consumer reads the data after it has seen it.
+// Everything else crosses a launch boundary.
 constexpr int NTH = 512;   // threads of every factorization workgroup (8 wavefronts)
 constexpr int NWAVE = NTH / 64;
 
@@ -93,37 +89,49 @@ template <bool CO, class R> __device__ __forceinline__ void cst(R* p, R v) {
     else *p = v;
 }
 
-// Panel flags sit one per 256-byte line so that pollers of different panels
-// do not share a memory channel.
+// Progress counters of a batch's models sit one per 256-byte line so that
+// pollers of different counters do not share a memory channel.
 constexpr long FLAG_STRIDE = 64;
 
-// thread 0 waits until flag i holds epoch (or an error is raised anywhere)
-__device__ inline bool wait_flag_bounded(const int* flags, long i, int epoch, long spin_limit, int* err,
-                                         int* ok_s) {
-    if (threadIdx.x == 0) {
-        long n = 0;
-        bool good = true;
-        const int* f = flags + i * FLAG_STRIDE;
-        while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != epoch) {
-            if (++n >= spin_limit) { good = false; break; }
-            if ((n & 63) == 0 && (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) & 1)) {
-                good = false;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(2);
-        }
-        if (!good) atomicOr(err, 1);
-        *ok_s = good;
-    }
-    __syncthreads();
-    return *ok_s != 0;
+__device__ __forceinline__ int peek(const int* c) {
+    return __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-__device__ inline void raise_flag(int* flags, long i, int epoch) {
-    __builtin_amdgcn_s_waitcnt(0);   // this wave's coherent stores have completed
+// one thread: polls *c until it is at least target (or an error is raised
+// anywhere); returns the value seen, below target on failure
+__device__ inline int poll_count(const int* c, int target, long spin_limit, int* err) {
+    for (long n = 0;; ++n) {
+        const int v = peek(c);
+        if (v >= target) return v;
+        if (n >= spin_limit || ((n & 63) == 63 && (peek(err) & 1))) {
+            atomicOr(err, 1);
+            return v;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
+
+// *c = value once every thread's stores have completed
+__device__ inline void publish(int* c, int value) {
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (threadIdx.x == 0)
-        __hip_atomic_store(flags + i * FLAG_STRIDE, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (threadIdx.x == 0) __hip_atomic_store(c, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__device__ __forceinline__ double lane_value(double x, int lane) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+    const unsigned lo = __builtin_amdgcn_readlane(unsigned(u), lane);
+    const unsigned hi = __builtin_amdgcn_readlane(unsigned(u >> 32), lane);
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+
+// threadIdx.x, opaque to the compiler: addresses formed from it are formed
+// where they are used.  In a loop over columns they would all be hoisted out,
+// and spilled.
+__device__ __forceinline__ int thread_index() {
+    int t = threadIdx.x;
+    __asm__ volatile("" : "+v"(t));
+    return t;
 }
 
 // ---- tile product C = X Y^T -------------------------------------------------
@@ -137,54 +145,69 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 // is fed Y as its A operand and X as its B operand (lane l: Y[16bj + l%16][k]
 // and X[16bi + l%16][k], k = k0 + l/16), so element e of lane l is
 // C[16bi + l%16][16bj + l/16 + 4e]: sixteen consecutive rows per column, which
-// makes the column-major tile stores coalesced.
+// makes the column-major tile stores coalesced.  Both blocks of a wavefront lie
+// in one block column, and the two wavefronts of a SIMD (wv and wv + 4) take
+// columns 3 and 0 or 2 and 1, which evens out product_ylower.
 template <> struct TileAcc<double> {
     d4 acc[2];
+    static __device__ __forceinline__ int block_col(int wv) { return (wv >> 1) ^ (wv < 4 ? 3 : 2); }
+    static __device__ __forceinline__ int block_row(int wv, int b) { return (2 * wv + b) & 3; }
     __device__ __forceinline__ void product(const double (*xs)[T], const double (*ys)[T]) {
-        const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+        const int t0 = thread_index(), l = t0 & 63, wv = t0 >> 6, bj = block_col(wv);
         acc[0] = d4{0.0, 0.0, 0.0, 0.0};
         acc[1] = d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
+#pragma unroll 8
         for (int k0 = 0; k0 < T; k0 += 4) {
             const int k = k0 + (l >> 4);
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const int blk = 2 * wv + b, bi = blk & 3, bj = blk >> 2;
-                acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ys[k][16 * bj + (l & 15)], xs[k][16 * bi + (l & 15)],
-                                                             acc[b], 0, 0, 0);
-            }
+            for (int b = 0; b < 2; ++b)
+                acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ys[k][16 * bj + (l & 15)],
+                                                             xs[k][16 * block_row(wv, b) + (l & 15)], acc[b], 0, 0, 0);
         }
     }
     // The same product for a lower-triangular Y (Y[col][k] = 0 for k > col):
     // the k-steps past the last column of the output block column add exact
-    // zeros and are skipped.  Both blocks of wavefront wv lie in block column
-    // wv / 2.
+    // zeros and are skipped.
     __device__ __forceinline__ void product_ylower(const double (*xs)[T], const double (*ys)[T]) {
-        const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
-        const int nkb = (__builtin_amdgcn_readfirstlane(wv) >> 1) + 1;   // 16-wide k blocks
+        const int t0 = thread_index(), l = t0 & 63, wv = __builtin_amdgcn_readfirstlane(t0 >> 6), bj = block_col(wv);
         acc[0] = d4{0.0, 0.0, 0.0, 0.0};
         acc[1] = d4{0.0, 0.0, 0.0, 0.0};
-        for (int kb = 0; kb < nkb; ++kb) {
+        // 16-wide k blocks, the next one's operands read beside the products
+        double y[4], x[4][2];
+        auto read = [&](int kb) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const int k = 16 * kb + 4 * t + (l >> 4);
+                y[t] = ys[k][16 * bj + (l & 15)];
 #pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    const int blk = 2 * wv + b, bi = blk & 3, bj = blk >> 2;
-                    acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ys[k][16 * bj + (l & 15)],
-                                                                 xs[k][16 * bi + (l & 15)], acc[b], 0, 0, 0);
-                }
+                for (int b = 0; b < 2; ++b) x[t][b] = xs[k][16 * block_row(wv, b) + (l & 15)];
             }
+        };
+        read(0);
+        for (int kb = 0; kb <= bj; ++kb) {
+            double yc[4], xc[4][2];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                yc[t] = y[t];
+                xc[t][0] = x[t][0];
+                xc[t][1] = x[t][1];
+            }
+            if (kb < bj) read(kb + 1);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(yc[t], xc[t][b], acc[b], 0, 0, 0);
         }
     }
     static constexpr int N = 8;   // entries per thread
     template <class F> __device__ __forceinline__ void each_i(F&& f) const {
-        const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+        const int t0 = thread_index(), l = t0 & 63, wv = t0 >> 6;
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            const int blk = 2 * wv + b, bi = blk & 3, bj = blk >> 2;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) f(16 * bi + (l & 15), 16 * bj + (l >> 4) + 4 * e, acc[b][e], 4 * b + e);
+            for (int e = 0; e < 4; ++e)
+                f(16 * block_row(wv, b) + (l & 15), 16 * block_col(wv) + (l >> 4) + 4 * e, acc[b][e], 4 * b + e);
         }
     }
     template <class F> __device__ __forceinline__ void each(F&& f) const {
@@ -253,22 +276,26 @@ struct LowerAcc {
         n = bi[1] >= 0 ? 2 : 1;
     }
     __device__ __forceinline__ void product(const double (*xs)[T], const double (*ys)[T]) {
-        const int l = threadIdx.x & 63;
+        const int l = thread_index() & 63;
         acc[0] = d4{0.0, 0.0, 0.0, 0.0};
         acc[1] = d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-        for (int k0 = 0; k0 < T; k0 += 4) {
-            const int k = k0 + (l >> 4);
-            acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ys[k][16 * bj[0] + (l & 15)], xs[k][16 * bi[0] + (l & 15)],
-                                                         acc[0], 0, 0, 0);
-            if (n == 2)
-                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ys[k][16 * bj[1] + (l & 15)],
-                                                             xs[k][16 * bi[1] + (l & 15)], acc[1], 0, 0, 0);
-        }
+        auto run = [&](auto two) {
+#pragma unroll 8
+            for (int k0 = 0; k0 < T; k0 += 4) {
+                const int k = k0 + (l >> 4);
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ys[k][16 * bj[0] + (l & 15)],
+                                                             xs[k][16 * bi[0] + (l & 15)], acc[0], 0, 0, 0);
+                if constexpr (decltype(two)::value)
+                    acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ys[k][16 * bj[1] + (l & 15)],
+                                                                 xs[k][16 * bi[1] + (l & 15)], acc[1], 0, 0, 0);
+            }
+        };
+        if (n == 2) run(std::true_type());
+        else run(std::false_type());
     }
     // f(row, col, value, i), i = 4 s + e
     template <class F> __device__ __forceinline__ void each_i(F&& f) const {
-        const int l = threadIdx.x & 63;
+        const int l = thread_index() & 63;
 #pragma unroll
         for (int s = 0; s < 2; ++s)
             if (s < n) {
@@ -277,6 +304,10 @@ struct LowerAcc {
             }
     }
 };
+
+// the symmetric product's accumulator at each precision
+template <class R> struct SymAcc : TileAcc<R> {};
+template <> struct SymAcc<double> : LowerAcc { static constexpr int N = 8; };
 
 // ---- D_K --------------------------------------------------------------------
 // The task takes the 64x64 tile S (lower part; the part above the diagonal is
@@ -341,7 +372,8 @@ template <int C> __device__ __forceinline__ double row_lane(double v) {   // v o
 }
 
 // Steps C .. 15: r is 1/d of pivot d = a[C] (lane C) to a relative error e
-// below 2^-23 and e2 = e + e^2, so that 1/d is r + r e2.  xs, dg: this lane's
+// below 2^-23 and e2 = e + e^2, so that 1/d is r + r e2; q = a[C] r.  xs, dg:
+// this lane's
 // entry of row 0 of the block and of the pivot columns; off: its byte offset
 // in a row of ys before the row's permutation.
 template <int C>
@@ -375,24 +407,25 @@ __device__ __forceinline__ void pivot_steps(double* a, double* x, double r, doub
     if constexpr (C < 15) pivot_steps<C + 1>(a, x, rn, qn, e2n, xs, ysb, off, dg);
 }
 
-struct NoHook {
-    __device__ void operator()() const {}
+struct NoSide {
+    __device__ void operator()(int, int) const {}
 };
 
-// tail_hook runs once before the last block column's pivot steps (every
-// thread): a caller issues loads there that it consumes after the task.  CO:
-// D and Linv are stored coherently, for readers in the same launch.
-template <bool CO = false, class Hook = NoHook, class O = double>
+// side(k, wv) runs on every wavefront in each block column's phase, on
+// wavefront 0 before the pivot steps and on the others beside them (after the
+// trailing blocks they may have).  LDS_ONLY: Linv goes to lds_out alone and D
+// stays in dd; the caller stores them.
+template <bool LDS_ONLY = false, class O = double, class Side = NoSide>
 __device__ __forceinline__ void diag_task(double (*xs)[T], double* ys, double* dd, DiagScratch<double>& sm,
                                           O* __restrict__ lout, double* __restrict__ piv, long Kt,
-                                          double* lds_out = nullptr, Hook tail_hook = Hook()) {
-    const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, rr = l & 15, lg = l >> 4;
+                                          O* lds_out = nullptr, Side side = Side()) {
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, rr = l & 15, lg = l >> 4;
     // block (q, p) of the elimination after block column m: A_qp (q >= p > m)
     // or B_pq (q <= m; its first contribution when q = m)
     // (the sixteen products are summed before they meet the entry, which
     // costs one rounding at its magnitude instead of four)
     auto trail = [&](int m, int p, int q) {
-        d4 old = {0.0, 0.0, 0.0, 0.0}, acc = {0.0, 0.0, 0.0, 0.0};
+        d4 old = {0.0, 0.0, 0.0, 0.0}, acc = old;
         if (q != m) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) old[e] = xs[16 * p + lg + 4 * e][16 * q + rr];
@@ -407,8 +440,8 @@ __device__ __forceinline__ void diag_task(double (*xs)[T], double* ys, double* d
     };
 #pragma unroll 1
     for (int k = 0; k < 4; ++k) {
-        if (k == 3) tail_hook();
         if (wv == 0) {
+            side(k, 0);
             const int base = 16 * k, row = 16 * ((k + lg) & 3) + rr;
             double a[16], x[16];
 #pragma unroll
@@ -422,22 +455,20 @@ __device__ __forceinline__ void diag_task(double (*xs)[T], double* ys, double* d
             const double d = row_lane<0>(a[0]), r = __builtin_amdgcn_rcp(d), e = __builtin_fma(-d, r, 1.0);
             pivot_steps<0>(a, x, r, a[0] * r, __builtin_fma(e, e, e), &xs[base][row],
                            reinterpret_cast<char*>(ys + base * T), (row ^ 4 * k) * 8, &sm.dg[0][rr]);
-            if (l < 16) {
-                const double dl = sm.dg[l][l];
-                dd[base + l] = dl;
-                cst<CO>(&piv[Kt * T + base + l], dl);
+            if (l < 16) dd[base + l] = sm.dg[l][l];
+        } else {
+            if (k == 1) {   // after block column 0: blocks of the columns 2 and 3
+                if (wv == 1) trail(0, 2, 0);
+                else if (wv == 2) trail(0, 2, 2);
+                else if (wv == 3) trail(0, 2, 3);
+                else if (wv == 5) trail(0, 3, 0);
+                else if (wv == 6) trail(0, 3, 3);
+            } else if (k == 2) {
+                if (wv == 1) trail(1, 3, 0);
+                else if (wv == 2) trail(1, 3, 1);
+                else if (wv == 3) trail(1, 3, 3);
             }
-        } else if (k == 1) {
-            // after block column 0: blocks of the columns 2 and 3
-            if (wv == 1) trail(0, 2, 0);
-            else if (wv == 2) trail(0, 2, 2);
-            else if (wv == 3) trail(0, 2, 3);
-            else if (wv == 5) trail(0, 3, 0);
-            else if (wv == 6) trail(0, 3, 3);
-        } else if (k == 2) {
-            if (wv == 1) trail(1, 3, 0);
-            else if (wv == 2) trail(1, 3, 1);
-            else if (wv == 3) trail(1, 3, 3);
+            side(k, wv);
         }
         __syncthreads();
         if (k < 3) {
@@ -445,12 +476,20 @@ __device__ __forceinline__ void diag_task(double (*xs)[T], double* ys, double* d
             __syncthreads();
         }
     }
-    for (int idx = threadIdx.x; idx < TT; idx += NTH) {
-        const int col = idx / T, row = idx % T;
-        const double v = (row >= col) ? ys[ysw(row, col)] : 0.0;
-        cst<CO>(&lout[idx], O(v));
-        if (lds_out) lds_out[idx] = v;
+    // Linv, column-major: all reads before the first store (one at a time took
+    // 1.5 us)
+    O v[TT / NTH];
+#pragma unroll
+    for (int i = 0; i < TT / NTH; ++i) {
+        const int idx = tid + NTH * i, col = idx / T, row = idx % T;
+        v[i] = O((row >= col) ? ys[ysw(row, col)] : 0.0);
     }
+#pragma unroll
+    for (int i = 0; i < TT / NTH; ++i) {
+        if (!LDS_ONLY) lout[tid + NTH * i] = v[i];
+        if (LDS_ONLY || lds_out) lds_out[tid + NTH * i] = v[i];
+    }
+    if (!LDS_ONLY && wv == 0) piv[Kt * T + l] = dd[l];
 }
 
 // FP32 tiles: the FP64 task on the tile widened in LDS, with Linv rounded once
@@ -459,18 +498,32 @@ __device__ __forceinline__ void diag_task(double (*xs)[T], double* ys, double* d
 // barrier per pivot made the FP32 column launch slower than the FP64 one.
 template <> struct DiagScratch<float> { double xd[T][T]; double yd[TT]; DiagScratch<double> in; };
 
-template <bool CO = false>
+template <bool LDS_ONLY = false, class Side = NoSide>
 __device__ __forceinline__ void diag_task(float (*xs)[T], float* /*ys*/, double* dd, DiagScratch<float>& sm,
-                                          float* __restrict__ lout, double* __restrict__ piv, long Kt) {
+                                          float* __restrict__ lout, double* __restrict__ piv, long Kt,
+                                          float* lds_out = nullptr, Side side = Side()) {
     for (int idx = threadIdx.x; idx < TT; idx += NTH) (&sm.xd[0][0])[idx] = double((&xs[0][0])[idx]);
     __syncthreads();
-    diag_task<CO>(sm.xd, sm.yd, dd, sm.in, lout, piv, Kt);
+    diag_task<LDS_ONLY>(sm.xd, sm.yd, dd, sm.in, lout, piv, Kt, lds_out, side);
 }
 
 // ---- staging ----------------------------------------------------------------
 template <bool CO, class R>
 __device__ __forceinline__ void stage(R (*dst)[T], const R* __restrict__ src) {
-    for (int idx = threadIdx.x; idx < TT; idx += NTH) dst[idx / T][idx % T] = cld<CO>(&src[idx]);
+    R buf[TT / NTH];   // all loads in flight before the first is used
+#pragma unroll
+    for (int i = 0; i < TT / NTH; ++i) buf[i] = cld<CO>(&src[threadIdx.x + NTH * i]);
+#pragma unroll
+    for (int i = 0; i < TT / NTH; ++i) (&dst[0][0])[threadIdx.x + NTH * i] = buf[i];
+}
+// A tile from LDS to memory by nthr threads, coherently, 16 bytes a store
+template <class R>
+__device__ __forceinline__ void put_tile(R* dst, const R (*src)[T], int i0, int nthr) {
+    typedef int i4 __attribute__((ext_vector_type(4)));
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(dst, 0, TT * sizeof(R), 0x00020000);
+#pragma unroll 4
+    for (int i = i0; i < int(TT * sizeof(R) / 16); i += nthr)
+        __builtin_amdgcn_raw_buffer_store_b128(reinterpret_cast<const i4*>(src)[i], rsrc, 16 * i, 0, 17);   // sc0 sc1
 }
 // dst[k][row] = src[k][row] * d[k]
 template <bool CO, class R>
@@ -554,141 +607,425 @@ __global__ void __launch_bounds__(NTH) k_tile_update(R* __restrict__ tiles, cons
 }
 
 // ---- fused schedule -----------------------------------------------------------
-// Launch K (K = -1 .. nt-2), m = min(w, nt-1-K) (0 for K = -1):
-//   workgroup 0          P_{K+1,K} and U_{K+1,K+1,K} in LDS only, then D_{K+1};
-//                        raises flag w once it has read A_{K+1,K}
-//   workgroups 1..m-1    P_{K+1+b,K}; raise flag b
-//   workgroup m          P_{K+1,K} again (the same arithmetic), stored once
-//                        flag w is up; raises flag 0
-//   the rest             U_{I,J,K} for the pairs other than (K+1,K+1), two tiles
-//                        of one tile row I per workgroup (they share L_IK)
-// Grid: m + 1 + sum_{r=1}^{m-1} ceil((r+1)/2) workgroups for m > 0 (194 at
-// m = 25, so that all of them are resident at once), 1 for m = 0.  Workgroup 0 neither
-// stores nor waits before its diagonal step.
+// One launch factors the band.  A tile keeps its entries in the registers of
+// the workgroup that owns it from the first update to the last (left-looking),
+// so it is read once and written once, and no launch boundary or flush lies
+// between the columns:
+//   chain      workgroup 0, column after column: P_{J,J-1} and U_{J,J,J-1} in
+//              LDS, D_J; Linv_J stays in LDS for the next panel
+//   tile(I, J) I - J >= 2: all updates, then P_{I,J}; (I, I-2) is handed to
+//              near(I) and corner(I) before its panel product
+//   near(I)    (I, I-1): all updates but the chain's, then handed to the chain.  For
+//              the last of them it forms P_{I,I-2} and P_{I-1,I-2} itself
+//   corner(I)  (I, I) likewise, with P_{I,I-2}
+// One column's critical path is then the chain's own P, U, D or half the loop
+// Linv_{J-2} -> near(J) -> chain -> Linv_J, whichever is longer.  The chain is:
+// 12.6 us a column whatever the band's width up to 25 tiles (panel 2.6, first
+// diagonal blocks 0.9, diagonal task 8.2, hand-over 0.9), against 21.2 us for
+// a launch per column whose workgroups loaded and stored every tile they
+// updated.  The workgroups of a band of 25 tiles need about 3 us a column of
+// the whole chip's matrix units, so they keep up.  Counters (zero
+// before the launch): P_ROW the columns of a tile row that its tile() tasks have
+// finished, P_LAST L_{J,J-1} stored, P_DIAG D_J and Linv_J stored, P_NEAR and
+// P_NEAR2 a row's two last tiles handed over, P_PART tile (I, I-2) handed over (in
+// slot (I, I) of tiles, which holds nothing else).
+// Workgroups are dispatched in index order and wait only on workgroups of
+// lower index and on the chain, which waits only on near and corner of the
+// column it has reached, whose own waits are on earlier columns; the lowest
+// unfinished workgroup is always resident, so every wait ends.  Waits are
+// bounded anyway.  Order: the chain, then by column J = 0, 1, ..: tile(J+2, J),
+// near(J+2), corner(J+2), tile(J+3, J) .. tile(J+m, J), m = min(w, nt-1-J)
+// (m + 1 workgroups, none for m < 2).
+// The band is assembled in tiles_t and the factor goes to tiles: no line of
+// tiles is read before it is written for good, and a tile's slot in tiles_t
+// receives the transposed factor tile when its owner has finished.
+constexpr long PSTRIDE = 16;   // a counter per 64 bytes
+enum { P_ROW = 0, P_LAST = 1, P_DIAG = 2, P_NEAR = 3, P_NEAR2 = 4, P_PART = 5, P_N = 6 };
+
+inline long factor_workgroups(long nt, int w) {
+    if (w < 2) return 1;
+    long g = 1 + std::max(0L, nt - w) * (w + 1);
+    for (long m = std::min<long>(w - 1, nt - 1); m >= 2; --m) g += m + 1;
+    return g;
+}
+
 template <class R>
-__global__ void __launch_bounds__(NTH) k_band_column(R* __restrict__ tiles, R* __restrict__ tiles_t,
-                                                     R* __restrict__ linv,
-                                                     double* __restrict__ piv, long K, int w, long nt,
-                                                     int* flags, int epoch, long spin_limit, int* err) {
+__global__ void __launch_bounds__(NTH) k_band_factor(R* __restrict__ tiles, R* __restrict__ tiles_t,
+                                                     R* __restrict__ linv, double* __restrict__ piv, int w, long nt,
+                                                     int* prog, long spin_limit, int* err) {
+    constexpr int N = TileAcc<R>::N, NS = TT / NTH;
     __shared__ R xs[T][T];
     __shared__ R ys[T][T];
-    __shared__ R zs[T][T];   // an update workgroup's second L_JK
+    __shared__ R zs[T][T];
+    __shared__ R lk[T][T];    // the chain's Linv_K
     __shared__ double dk[T];
-    // wait results: one slot per flag waited on
-    __shared__ int ok_s[3];
-    const long m = (K < 0) ? 0 : ((nt - 1 - K < w) ? nt - 1 - K : w);
-    const long b = blockIdx.x;
-    if (m > 0 && threadIdx.x < T) dk[threadIdx.x] = piv[K * T + threadIdx.x];
-    if (b == 0) {
-        __shared__ DiagScratch<R> sm;
-        const long D = K + 1;
-        const R* dtile = tiles + tile_index(D, D, w) * TT;
-        if (m == 0) {
-            stage<false>(xs, dtile);
-            __syncthreads();
-            diag_task(xs, &ys[0][0], dk, sm, linv + D * (long)TT, piv, D);
-            return;
-        }
-        R pre[TileAcc<R>::N];
-        if constexpr (std::is_same<R, double>::value) {
-            LowerAcc pos;
-            pos.each_i([&](int row, int col, double, int i) { pre[i] = dtile[col * T + row]; });
-        } else {
-            gather_tile(dtile, pre);
-        }
-        stage<false>(xs, tiles + tile_index(D, K, w) * TT);
-        stage<false>(ys, linv + K * (long)TT);
-        raise_flag(flags, w, epoch);   // A_{K+1,K} has been read (includes the barrier)
-        TileAcc<R> acc;
-        acc.product_ylower(xs, ys);   // Linv_K is lower triangular
+    __shared__ R rdk[T];      // 1 / D_K
+    __shared__ DiagScratch<R> sm;
+    __shared__ int seen_s[2][2];
+    __shared__ R zd[std::is_same<R, double>::value ? 10 : 1][256];   // the chain's next A_JJ, by 16x16 blocks
+    __shared__ int got_s[4], drained_s[2];
+    // 4 * block row + block column of lower 16x16 block b, by columns
+    auto dblk = [](int b) { return int(0xFEAD95C840ull >> 4 * b & 15); };
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto cnt = [&](int kind, long i) { return prog + (kind * nt + i) * PSTRIDE; };
+    auto tile = [&](R* base, long I, long J) { return base + tile_index(I, J, w) * TT; };
+    // Waits until both counters have reached the target; returns the smaller
+    // value, below the target after an error.  seen_s alternates, so that a
+    // wait's values are not overwritten before every thread has read them.
+    int par = 0;
+    auto wait2 = [&](const int* c0, const int* c1, int target) {
+        if (tid == 0) seen_s[par][0] = poll_count(c0, target, spin_limit, err);
+        if (tid == 64) seen_s[par][1] = poll_count(c1, target, spin_limit, err);
         __syncthreads();
-        // (L D, L) of L = P_{K+1,K} to LDS for U_{K+1,K+1,K}
+        const int v = min(seen_s[par][0], seen_s[par][1]);
+        par ^= 1;
+        return v;
+    };
+    auto wait1 = [&](const int* c, int target) {
+        if (tid == 0) seen_s[par][0] = poll_count(c, target, spin_limit, err);
+        __syncthreads();
+        const int v = seen_s[par][0];
+        par ^= 1;
+        return v >= target;
+    };
+    auto load_co = [&](R* buf, const R* src) {
+#pragma unroll
+        for (int i = 0; i < NS; ++i) buf[i] = cld<true>(&src[tid + NTH * i]);
+    };
+    auto to_lds = [&](R (*dst)[T], const R* buf) {
+#pragma unroll
+        for (int i = 0; i < NS; ++i) dst[wv + NWAVE * i][lane] = buf[i];
+    };
+    // dst = buf scaled by column with D_K, of which this lane holds entry `lane`
+    auto to_lds_scaled = [&](R (*dst)[T], const R* buf, double d) {
+#pragma unroll
+        for (int i = 0; i < NS; ++i) dst[wv + NWAVE * i][lane] = buf[i] * R(lane_value(d, wv + NWAVE * i));
+    };
+    // ys = Linv_K and dk, rdk = D_K, 1 / D_K, in the coherent copies
+    auto stage_linv = [&](long K) {
+        if (tid < T) {
+            const double d = cld<true>(&piv[K * T + tid]);
+            dk[tid] = d;
+            rdk[tid] = R(1) / R(d);
+        }
+        stage<true>(ys, linv + K * (long)TT);
+    };
+
+    if (blockIdx.x == 0) {
+        if (tid < 2) drained_s[tid] = 0;
+        // A column's tiles sit in the pair (a0, a1): A_{J,J-1} and Linv_{J-1},
+        // then, once the panel product has read them, the diagonal task's
+        // tile and rows.  The other pair holds the panel (L D, L) until the
+        // diagonal update is done, in the first phase of the task, and
+        // receives A_{J+1,J} (as soon as near(J+1) has handed it over) and
+        // Linv_J for the next column.
+        R (*a0)[T] = xs, (*a1)[T] = ys, (*b0)[T] = zs, (*b1)[T] = lk;
+        constexpr bool D64 = std::is_same<R, double>::value;
+        for (long J = 0; J < nt; ++J) {
+            const bool handed = J >= 2 && w >= 2;              // near(J) exists
+            const bool hands = J + 1 >= 2 && w >= 2;           // near(J+1) exists, if row J+1 does
+            const R* dt = tile(tiles_t, J, J);
+            bool got2 = false;
+            if (J == 0) {
+                stage<false>(a0, dt);
+                __syncthreads();
+            } else {
+                if (wv >= 4) {   // the last of these sees D_{J-1} and Linv_{J-1} complete in memory
+                    put_tile(linv + (J - 1) * (long)TT, a1, tid - NTH / 2, NTH / 2);
+                    if (wv == 4) cst<true>(&piv[(J - 1) * T + lane], dk[lane]);
+                    __builtin_amdgcn_s_waitcnt(0);
+                    if (lane == 0 && atomicAdd(&drained_s[0], 1) == 4 * int(J) - 1)
+                        __hip_atomic_store(cnt(P_DIAG, J - 1), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                }
+                const int got = got_s[0] & got_s[1] & got_s[2] & got_s[3];
+                got2 = got & 2;
+                if (!(got & 1)) {
+                    if (handed) {
+                        if (!wait1(cnt(P_NEAR, J), 1)) return;
+                        stage<true>(a0, tile(tiles_t, J, J - 1));
+                    } else {
+                        stage<false>(a0, tile(tiles_t, J, J - 1));
+                    }
+                    __syncthreads();
+                }
+                TileAcc<R> acc;
+                acc.product_ylower(a0, a1);
+                R* tout = tile(tiles_t, J, J - 1);
+                const bool own_t = !hands || J + 1 >= nt;      // else near(J+1) stores the transposed tile
+                acc.each([&](int row, int col, R v) {
+                    const R p = v * rdk[col];
+                    b0[col][row] = p * R(dk[col]);
+                    b1[col][row] = p;
+                    if (own_t) tout[row * T + col] = p;
+                });
+                __syncthreads();
+                if (handed && !got2 && !wait1(cnt(P_NEAR2, J), 1)) return;
+            }
+            // block b of the ten lower 16x16 blocks of A_JJ - U_{J,J,J-1}, one wavefront
+            auto diag_block = [&](int b) {
+                const int lane = thread_index() & 63;
+                const int bi = dblk(b) >> 2, bj = dblk(b) & 3;
+                R pre[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int row = 16 * bi + (lane & 15), col = 16 * bj + (lane >> 4) + 4 * e;
+                    pre[e] = got2 ? zd[b][64 * e + lane] : handed ? cld<true>(&dt[col * T + row]) : dt[col * T + row];
+                }
+                d4 u = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+                for (int k0 = 0; k0 < T; k0 += 4) {
+                    const int k = k0 + (lane >> 4);
+                    u = __builtin_amdgcn_mfma_f64_16x16x4f64(b1[k][16 * bj + (lane & 15)], b0[k][16 * bi + (lane & 15)], u,
+                                                            0, 0, 0);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a0[16 * bj + (lane >> 4) + 4 * e][16 * bi + (lane & 15)] = pre[e] - u[e];
+            };
+            if (J > 0) {
+                if constexpr (D64) {
+                    if (wv < 4) diag_block(wv);   // the first block column; the rest beside its pivots
+                    else put_tile(tile(tiles, J, J - 1), b1, tid - NTH / 2, NTH / 2);
+                } else {
+                    TileAcc<R> u;
+                    u.product(b0, b1);
+                    u.each([&](int row, int col, R v) {
+                        const R p = handed ? cld<true>(&dt[col * T + row]) : dt[col * T + row];
+                        a0[col][row] = p - v;
+                    });
+                    if (wv >= 4) put_tile(tile(tiles, J, J - 1), b1, tid - NTH / 2, NTH / 2);
+                }
+                __syncthreads();
+            }
+            // Beside the pivots: the rest of the diagonal update, then
+            // wavefronts 3, 5, 6 and 7 fetch the next column's tiles as they
+            // are handed over (loaded in one phase, written to LDS in a later
+            // one; got: 1, 2 loaded, 4, 8 written).
+            int got = 0;
+            const int part = wv == 3 ? 0 : wv - 4;
+            const bool fetcher = J + 1 < nt && (wv == 3 || wv > 4);
+            R buf1[16], buf2[10];
+            auto settle = [&](int ln) {
+                if ((got & 5) == 1) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) b0[16 * part + i][ln] = buf1[i];
+                    got |= 4;
+                }
+                if (D64 && (got & 10) == 2) {
+#pragma unroll
+                    for (int i = 0; i < 10; ++i) zd[0][(10 * part + i) * 64 + ln] = buf2[i];
+                    got |= 8;
+                }
+            };
+            diag_task<true>(a0, &a1[0][0], dk, sm, (R*)nullptr, piv, J, &b1[0][0], [&](int k, int v) {
+                if (v == 0) return;
+                const int ln = thread_index() & 63;
+                if (k == 0) {
+                    if (J > 0 && v >= 4) {   // the panel is complete in memory
+                        __builtin_amdgcn_s_waitcnt(0);
+                        if (ln == 0 && atomicAdd(&drained_s[1], 1) == 4 * int(J) - 1)
+                            __hip_atomic_store(cnt(P_LAST, J), int(J), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    }
+                    if constexpr (D64)
+                        if (J > 0 && v != 4) diag_block(v < 4 ? 3 + v : 2 + v);
+                    return;
+                }
+                if (!fetcher) return;
+                settle(ln);
+                auto there = [&](int kind) { return !hands || __builtin_amdgcn_readfirstlane(peek(cnt(kind, J + 1))) != 0; };
+                if (!(got & 1) && there(P_NEAR)) {
+                    const R* src = tile(tiles_t, J + 1, J);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const R* q = &src[(16 * part + i) * T + ln];
+                        buf1[i] = hands ? cld<true>(q) : *q;
+                    }
+                    got |= 1;
+                }
+                if (D64 && !(got & 2) && there(P_NEAR2)) {
+                    const R* src = tile(tiles_t, J + 1, J + 1);
+#pragma unroll
+                    for (int i = 0; i < 10; ++i) {
+                        const int f = 10 * part + i, b = f >> 2, e = f & 3;
+                        const R* q = &src[(16 * (dblk(b) & 3) + (ln >> 4) + 4 * e) * T + 16 * (dblk(b) >> 2) + (ln & 15)];
+                        buf2[i] = hands ? cld<true>(q) : *q;
+                    }
+                    got |= 2;
+                }
+            });
+            if (fetcher) settle(lane);
+            if (tid < T) rdk[tid] = R(1) / R(dk[tid]);
+            if (lane == 0 && (wv == 3 || wv > 4)) got_s[part] = got >> 2;
+            __syncthreads();
+            R (*p0)[T] = a0, (*p1)[T] = a1;
+            a0 = b0;
+            a1 = b1;
+            b0 = p0;
+            b1 = p1;
+        }
+        put_tile(linv + (nt - 1) * (long)TT, a1, tid, NTH);
+        if (tid < T) cst<true>(&piv[(nt - 1) * T + tid], dk[tid]);
+        return;
+    }
+
+    // column and place in it
+    long t = long(blockIdx.x) - 1, J, m = w;
+    const long nfull = nt > w ? nt - w : 0;
+    if (t < nfull * (w + 1)) {
+        J = t / (w + 1);
+        t -= J * (w + 1);
+    } else {
+        t -= nfull * (w + 1);
+        J = nfull;
+        m = nt - 1 - J;
+        while (t >= m + 1) {
+            t -= m + 1;
+            ++J;
+            --m;
+        }
+    }
+    R xr[NS], yr[NS];
+    double dr = 0.0;
+    if (t == 2) {
+        const long I = J + 2;
+        SymAcc<R> sym;
+        R c[SymAcc<R>::N];
+        R* t2 = tile(tiles_t, I, I);
+        sym.each_i([&](int row, int col, R, int i) { c[i] = t2[col * T + row]; });
+        long K = I - w > 0 ? I - w : 0;
+        int ready = 0;
+        auto fetch = [&] {
+            load_co(xr, tile(tiles, I, K));
+            dr = cld<true>(&piv[K * T + lane]);
+        };
+        if (K < J) {
+            ready = wait2(cnt(P_ROW, I), cnt(P_ROW, I), int(K + 1));
+            if (ready < K + 1) return;
+            fetch();
+        }
+        while (K < J) {
+            to_lds_scaled(xs, xr, dr);
+            to_lds(ys, xr);
+            __syncthreads();
+            ++K;
+            const bool next = K < J && K < ready;
+            if (next) fetch();
+            sym.product(xs, ys);
+            sym.each_i([&](int, int, R v, int i) { c[i] -= v; });
+            if (next || K >= J) {
+                __syncthreads();
+            } else {
+                ready = wait2(cnt(P_ROW, I), cnt(P_ROW, I), int(K + 1));
+                if (ready < K + 1) return;
+                fetch();
+            }
+        }
+        if (!wait1(cnt(P_PART, I), 1)) return;
+        stage<true>(xs, tile(tiles, I, I));
+        if (!wait1(cnt(P_DIAG, J), 1)) return;
+        stage_linv(J);
+        __syncthreads();
+        TileAcc<R> acc;
+        acc.product_ylower(xs, ys);
+        __syncthreads();
         acc.each([&](int row, int col, R v) {
-            const R lv = v * (R(1) / R(dk[col]));
-            xs[col][row] = lv * R(dk[col]);
-            ys[col][row] = lv;
+            const R p = v * rdk[col];
+            xs[col][row] = p * R(dk[col]);
+            ys[col][row] = p;
         });
         __syncthreads();
-        // U_{K+1,K+1,K} is symmetric and the diagonal task reads only its
-        // lower part
-        if constexpr (std::is_same<R, double>::value) {
-            LowerAcc u;
-            u.product(xs, ys);
-            __syncthreads();
-            u.each_i([&](int row, int col, double v, int i) { xs[col][row] = pre[i] - v; });
-        } else {
-            acc.product(xs, ys);
-            __syncthreads();
-            acc.each_i([&](int row, int col, R v, int i) { xs[col][row] = pre[i] - v; });
-        }
+        sym.product(xs, ys);
+        sym.each_i([&](int row, int col, R v, int i) { cst<true>(&t2[col * T + row], c[i] - v); });
+        publish(cnt(P_NEAR2, I), 1);
+        return;
+    }
+
+    // tile(I, J), and near(I) up to its last update
+    const bool near = t == 1;
+    const long I = J + (t < 2 ? 2 : t), C = near ? I - 1 : J;   // the workgroup's tile is (I, C)
+    R* tt = tile(tiles_t, I, C);
+    R c[N];
+    gather_tile(tt, c);
+    long K = I - w > 0 ? I - w : 0;
+    int ready = 0;
+    auto fetch = [&] {
+        load_co(xr, tile(tiles, I, K));
+        load_co(yr, tile(tiles, C, K));
+        dr = cld<true>(&piv[K * T + lane]);
+    };
+    // L_{C,C-1} is the chain's
+    auto wait_for = [&] { return ready = wait2(cnt(P_ROW, I), cnt(K + 1 == C ? P_LAST : P_ROW, C), int(K + 1)); };
+    if (K < J) {
+        if (wait_for() < K + 1) return;
+        fetch();
+    }
+    while (K < J) {
+        to_lds_scaled(xs, xr, dr);
+        to_lds(ys, yr);
         __syncthreads();
-        diag_task(xs, &ys[0][0], dk, sm, linv + D * (long)TT, piv, D);
-        return;
-    }
-    __syncthreads();   // dk
-    if (b <= m) {
-        const long pb = (b == m) ? 0 : b;
-        const long I = K + 1 + pb;
-        R* tile = tiles + tile_index(I, K, w) * TT;
-        R* ttile = tiles_t + tile_index(I, K, w) * TT;
-        // stage (workgroup m then waits until workgroup 0 has read the tile
-        // before overwriting it), product, coherent stores, flag; the
-        // transposed copy for the backward sweep is stored after the flag
-        stage<false>(xs, tile);
-        stage<false>(ys, linv + K * (long)TT);
-        bool ok = true;
-        if (pb == 0) ok = wait_flag_bounded(flags, w, epoch, spin_limit, err, &ok_s[0]);
-        else __syncthreads();
+        ++K;
+        const bool next = K < J && K < ready;   // known to be there: load it during the product
+        if (next) fetch();
         TileAcc<R> acc;
-        acc.product_ylower(xs, ys);   // Linv_K is lower triangular
-        if (ok) acc.each([&](int row, int col, R v) { cst<true>(&tile[col * T + row], v * (R(1) / R(dk[col]))); });
-        raise_flag(flags, pb, epoch);
-        if (ok) acc.each([&](int row, int col, R v) { ttile[row * T + col] = v * (R(1) / R(dk[col])); });
-        return;
-    }
-    // row r >= 1 of the update triangle holds ceil((r+1)/2) workgroups
-    long t = b - (m + 1), r = 1;
-    for (long c = (r + 2) / 2; t >= c; c = (r + 2) / 2) {
-        t -= c;
-        ++r;
-    }
-    const long s0 = 2 * t, ns = (s0 + 1 <= r) ? 2 : 1;
-    // the (up to three) panel flags of the pair, polled side by side: lane i
-    // of wavefront 0 polls flag i, so the waits cost one round trip together
-    if (threadIdx.x < 3) {
-        const int i = threadIdx.x;
-        const long f = (i == 0) ? r : s0 + (i - 1);
-        const bool need = (i == 0) || (i - 1 < ns && f != r);
-        bool good = true;
-        if (need) {
-            const int* fp = flags + f * FLAG_STRIDE;
-            long n = 0;
-            while (__hip_atomic_load(fp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != epoch) {
-                if (++n >= spin_limit) { good = false; break; }
-                if ((n & 63) == 0 && (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) & 1)) {
-                    good = false;
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(2);
-            }
-            if (!good) atomicOr(err, 1);
+        acc.product(xs, ys);
+        acc.each_i([&](int, int, R v, int i) { c[i] -= v; });
+        if (next || K >= J) {
+            __syncthreads();
+        } else {
+            if (wait_for() < K + 1) return;
+            fetch();
         }
-        ok_s[i] = good;
     }
-    __syncthreads();
-    if (!(ok_s[0] && ok_s[1] && ok_s[2])) return;
-    const long I = K + 1 + r;
-    // L_IK D_K and both L_JK staged together
-    stage_scaled<true>(xs, tiles + tile_index(I, K, w) * TT, dk);
-    stage<true>(ys, tiles + tile_index(K + 1 + s0, K, w) * TT);
-    if (ns == 2) stage<true>(zs, tiles + tile_index(K + 2 + s0, K, w) * TT);
-    __syncthreads();
-    for (long j = 0; j < ns; ++j) {
-        TileAcc<R> acc;
-        acc.product(xs, j == 0 ? ys : zs);
-        R* out = tiles + tile_index(I, K + 1 + s0 + j, w) * TT;
-        acc.each([&](int row, int col, R v) { out[col * T + row] -= v; });
+    TileAcc<R> acc;
+    if (!near) {
+        if (t == 0) {
+            R* part = tile(tiles, I, I);
+            acc.each_i([&](int row, int col, R, int i) { cst<true>(&part[col * T + row], c[i]); });
+            publish(cnt(P_PART, I), 1);
+        }
+        acc.each_i([&](int row, int col, R, int i) { xs[col][row] = c[i]; });
+        if (!wait1(cnt(P_DIAG, J), 1)) return;
+        stage_linv(J);
+        __syncthreads();
+        acc.product_ylower(xs, ys);
+        R* out = tile(tiles, I, J);
+        acc.each_i([&](int row, int col, R v, int i) {
+            c[i] = v * rdk[col];
+            cst<true>(&out[col * T + row], c[i]);
+        });
+        publish(cnt(P_ROW, I), int(J + 1));
+        acc.each_i([&](int row, int col, R, int i) { tt[row * T + col] = c[i]; });
+        return;
     }
+    // near(I): (I, I-2) as its owner and (I-1, I-2) as the chain got them
+    R* t1 = tile(tiles_t, I - 1, J);
+    if (!wait1(cnt(P_PART, I), 1)) return;
+    stage<true>(xs, tile(tiles, I, I));
+    if (I > 2) {
+        if (!wait1(cnt(P_NEAR, I - 1), 1)) return;
+        stage<true>(zs, t1);
+    } else {
+        stage<false>(zs, t1);
+    }
+    if (!wait1(cnt(P_DIAG, J), 1)) return;
+    stage_linv(J);
+    __syncthreads();
+    TileAcc<R> acc1;
+    acc.product_ylower(xs, ys);
+    acc1.product_ylower(zs, ys);
+    __syncthreads();
+    R lv1[N];
+    acc.each([&](int row, int col, R v) { xs[col][row] = v * rdk[col] * R(dk[col]); });
+    acc1.each_i([&](int row, int col, R v, int i) {
+        lv1[i] = v * rdk[col];
+        ys[col][row] = lv1[i];
+    });
+    __syncthreads();
+    acc.product(xs, ys);
+    acc.each_i([&](int row, int col, R v, int i) { cst<true>(&tt[col * T + row], c[i] - v); });
+    publish(cnt(P_NEAR, I), 1);
+    // the chain has read (I-1, I-2) once it has published row I-1
+    if (!wait1(cnt(P_LAST, I - 1), 1)) return;
+    acc.each_i([&](int row, int col, R, int i) { t1[row * T + col] = lv1[i]; });
 }
 
 // ---- pipelined sweeps ---------------------------------------------------------
@@ -1463,29 +1800,9 @@ enum { C_DIAG = 0, C_P1 = 1, C_U21 = 2, C_U22 = 3 };
 
 // thread 0 waits until *c >= target (or an error is raised anywhere)
 __device__ inline bool wait_count(const int* c, int target, long spin_limit, int* err, int* ok_s) {
-    if (threadIdx.x == 0) {
-        long n = 0;
-        bool good = true;
-        while (__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) < target) {
-            if (++n >= spin_limit) { good = false; break; }
-            if ((n & 63) == 0 && (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) & 1)) {
-                good = false;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(2);
-        }
-        if (!good) atomicOr(err, 1);
-        *ok_s = good;
-    }
+    if (threadIdx.x == 0) *ok_s = poll_count(c, target, spin_limit, err) >= target;
     __syncthreads();
     return *ok_s != 0;
-}
-
-// *c = value once every thread's stores have completed
-__device__ inline void publish(int* c, int value) {
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(c, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ void __launch_bounds__(NTH) k_band_factor_models(double* __restrict__ tiles, double* __restrict__ linv,
@@ -1557,8 +1874,8 @@ __global__ void __launch_bounds__(NTH) k_band_factor_models(double* __restrict__
             __syncthreads();
         }
         staged = false;
-        diag_task(xs, ys, dd, sm, linv + K * (long)TT, piv, K, &lk[0][0], [&] {
-            if (pre) {
+        diag_task(xs, ys, dd, sm, linv + K * (long)TT, piv, K, &lk[0][0], [&](int k, int) {
+            if (pre && k == 3) {
                 const double* t1 = tiles + tile_index(K + 1, K, w) * TT;
 #pragma unroll
                 for (int i = 0; i < TT / NTH; ++i) pa[i] = t1[threadIdx.x + NTH * i];
@@ -1875,17 +2192,15 @@ void BandLDLT<R>::setup(long n_, long bandwidth, hipStream_t s_) {
     xw = dalloc<double>(size_t(nt) * T);
     yw = dalloc<double>(size_t(nt) * T);
     flag = dalloc<int>(1);
-    pflags = dalloc<int>(size_t(w + 1) * FLAG_STRIDE);
-    CB_CHECK(hipMemsetAsync(pflags, 0, sizeof(int) * size_t(w + 1) * FLAG_STRIDE, s));
+    prog = dalloc<int>(size_t(P_N * nt * PSTRIDE));
     CB_CHECK(hipMemsetAsync(flag, 0, sizeof(int), s));
-    cepoch = 0;
     piv_host.resize(size_t(n));
     CB_CHECK(hipStreamSynchronize(s));
 }
 
 template <class R>
 void BandLDLT<R>::release() {
-    void* ps[] = {tiles, tiles_t, linv, mch, gch, piv, xw, yw, flag, pflags, l2, w2, bp, b2, v2, zp, l3, b3, bq, zq};
+    void* ps[] = {tiles, tiles_t, linv, mch, gch, piv, xw, yw, flag, prog, l2, w2, bp, b2, v2, zp, l3, b3, bq, zq};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     tiles = nullptr; tiles_t = nullptr; linv = nullptr; piv = nullptr; xw = nullptr; yw = nullptr; flag = nullptr;
@@ -1893,45 +2208,35 @@ void BandLDLT<R>::release() {
     l2 = nullptr; w2 = nullptr; bp = nullptr;
     b2 = nullptr; v2 = nullptr; zp = nullptr;
     l3 = nullptr; b3 = nullptr; bq = nullptr; zq = nullptr;
-    pflags = nullptr;
+    prog = nullptr;
     clock.release();
 }
 
 template <class R>
 int BandLDLT<R>::factor(const Dev& d) {
-    CB_CHECK(hipMemsetAsync(tiles, 0, sizeof(R) * size_t(nt) * (w + 1) * TT, s));
+    // the fused schedule takes the matrix from tiles_t
+    R* band = split ? tiles : tiles_t;
+    CB_CHECK(hipMemsetAsync(band, 0, sizeof(R) * size_t(nt) * (w + 1) * TT, s));
     CB_CHECK(hipMemsetAsync(flag, 0, sizeof(int), s));
     if (src32)
-        hipLaunchKernelGGL((k_band_from_bsr<R, float>), dim3(int((d.nslot + 255) / 256)), dim3(256), 0, s, tiles,
+        hipLaunchKernelGGL((k_band_from_bsr<R, float>), dim3(int((d.nslot + 255) / 256)), dim3(256), 0, s, band,
                            d.K32, d.rowptr, d.colidx, d.eq_of_slot, d.nj, d.bs, w, flag);
     else
-        hipLaunchKernelGGL((k_band_from_bsr<R>), dim3(int((d.nslot + 255) / 256)), dim3(256), 0, s, tiles,
+        hipLaunchKernelGGL((k_band_from_bsr<R>), dim3(int((d.nslot + 255) / 256)), dim3(256), 0, s, band,
                            d.K, d.rowptr, d.colidx, d.eq_of_slot, d.nj, d.bs, w, flag);
     if (nt * T > n)
-        hipLaunchKernelGGL((k_band_pad<R>), dim3(1), dim3(T), 0, s, tiles, n, nt, w);
+        hipLaunchKernelGGL((k_band_pad<R>), dim3(1), dim3(T), 0, s, band, n, nt, w);
     CB_CHECK(hipGetLastError());
     if (!split) {
-        if (cepoch + nt + 1 >= (1 << 30)) {
-            CB_CHECK(hipMemsetAsync(pflags, 0, sizeof(int) * size_t(w + 1) * FLAG_STRIDE, s));
-            cepoch = 0;
-        }
         const long spin_limit = 1L << 22;
+        CB_CHECK(hipMemsetAsync(prog, 0, sizeof(int) * size_t(P_N * nt * PSTRIDE), s));
         const bool tk_column = clock.on(KT_COLUMN);
         if (tk_column) {
             clock.launches[KT_COLUMN] += nt;
             clock.begin(KT_COLUMN, s, nt);
         }
-        for (long K = -1; K < nt - 1; ++K) {
-            const long m = (K < 0) ? 0 : std::min<long>(w, nt - 1 - K);
-            long grid = 1;
-            if (m > 0) {
-                grid = m + 1;
-                for (long rr = 1; rr < m; ++rr) grid += (rr + 2) / 2;
-            }
-            cepoch += 1;
-            hipLaunchKernelGGL((k_band_column<R>), dim3(int(grid)), dim3(NTH), 0, s, tiles, tiles_t, linv, piv, K, w,
-                               nt, pflags, cepoch, spin_limit, flag + 0);
-        }
+        hipLaunchKernelGGL((k_band_factor<R>), dim3(unsigned(factor_workgroups(nt, w))), dim3(NTH), 0, s, tiles,
+                           tiles_t, linv, piv, w, nt, prog, spin_limit, flag);
         if (tk_column) clock.end(s);
     } else {
         for (long Kt = 0; Kt < nt; ++Kt) {
@@ -1993,7 +2298,7 @@ int BandLDLT<R>::factor(const Dev& d) {
     CB_CHECK(hipMemcpyAsync(piv_host.data(), piv, sizeof(double) * size_t(n), hipMemcpyDeviceToHost, s));
     CB_CHECK(hipStreamSynchronize(s));
     clock.collect();
-    if (bad & 1) throw DeviceError("band factorization: a panel wait exceeded its bound");
+    if (bad & 1) throw DeviceError("band factorization: a wait exceeded its bound");
     if (bad & 2) return 2;
     for (long i = 0; i < n; ++i)
         if (piv_host[i] == 0.0 || !std::isfinite(piv_host[i])) return 1;

@@ -50,7 +50,7 @@ struct RunOptions {
     int max_steps = 1 << 30;
     int keep_d = 1;         // copy d to the host at every converged step
     int kernel_timing = 0;  // KT_* bitmask of band kernels timed with HIP events
-    int factor_schedule = 0;  // 0 fused launch per tile column, 1 split diag/panel/update launches
+    int factor_schedule = 0;  // 0 one fused launch, 1 split diag/panel/update launches per tile column
     int kernel_timing_every = 1;  // time every n-th launch of a timed family
     int sweep_schedule = 0;       // 0 sweeps with the chain matrices, 1 the two-product row step,
                                   // 2 both sweeps on the look-ahead system (rows two back)

@@ -89,9 +89,9 @@ typedef struct {
 } cb_options;
 
 /* Schedules of the band LDL^T factorization (same tile arithmetic, bitwise
- * the same result): one fused launch per tile column whose workgroups hand
- * the panels to the updates through flags, or a diag, a panel and an update
- * launch per tile column (for timing the tile tasks one by one). */
+ * the same result): one launch whose workgroups hand the tiles to each other
+ * through progress counters, or a diag, a panel and an update launch per tile
+ * column (for timing the tile tasks one by one). */
 enum { CB_FACTOR_FUSED = 0, CB_FACTOR_SPLIT = 1 };
 
 /* Schedules of the band solves' forward and backward sweeps (the same
@@ -112,7 +112,7 @@ enum { CB_SWEEP_CHAIN = 0, CB_SWEEP_ROWS = 1, CB_SWEEP_LOOK2 = 2, CB_SWEEP_LOOK3
 enum { CB_GEN_BASE = 0, CB_GEN_I = 1, CB_GEN_IP = 2 };
 
 /* Kernel families of the band solver (timed with HIP events on their stream):
- * the fused per-column factorization launch, the diag/panel/update launches
+ * the fused factorization launch (per tile column), the diag/panel/update launches
  * of the split schedule, the forward and backward sweeps, and the launch that
  * forms the sweeps' chain matrices after a factorization. */
 enum { CB_KT_COLUMN = 0, CB_KT_DIAG = 1, CB_KT_PANEL = 2, CB_KT_UPDATE = 3, CB_KT_FWD = 4, CB_KT_BWD = 5,
