@@ -11,7 +11,7 @@ namespace cb {
 // Kernel families of the band solver whose launches can be timed with HIP
 // events: KT_COLUMN is the fused factorization, per tile column; KT_DIAG,
 // KT_PANEL and KT_UPDATE are the launches of the split schedule.
-// KT_PREP times the launch that forms the sweeps' chain matrices after a
+// KT_PREP times the launches that form the sweeps' block matrices after a
 // factorization.
 enum { KT_COLUMN = 0, KT_DIAG = 1, KT_PANEL = 2, KT_UPDATE = 3, KT_FWD = 4, KT_BWD = 5, KT_PREP = 6, KT_N = 7 };
 
@@ -55,28 +55,19 @@ struct BandLDLT {
     R* tiles_t = nullptr;    // the factor's off-diagonal tiles transposed (row-major), for the backward sweep
     R* linv = nullptr;
     double* piv = nullptr;   // pivots D (padded to nt*T)
-    // chain matrices of the sweeps, formed after each factorization: M_I =
-    // Linv_I L_{I,I-1} and G_I = L_{I+1,I} Linv_I, [nt][T*T] each
+    // block sweeps: the inverses of the factor's 4 x 4 diagonal tile blocks below
+    // their diagonal tiles [blocks][6], and the links M_B = Linv_B L_{B,B-1} and G_B =
+    // Linv_B^T L_{B+1,B}^T [nt][4], formed after each factorization; the
+    // right-hand side [nt * 64] and the helpers' partial sums; allocated at the
+    // first factorization that needs them
+    bool chained = true;     // block sweeps (default) or the two-product row step
+    // a band of at most one block of four tile rows takes the row step
+    bool blocked() const { return chained && nt > 4; }
+    R* lb = nullptr;
     R* mch = nullptr;
     R* gch = nullptr;
-    bool chained = true;     // sweeps with the chain matrices (default) or the two-product row step
-    // the forward sweep two rows ahead (with chained): L' and W of the
-    // look-ahead system [nt][w] and [nt] tiles, b' [nt * 64]; allocated at the
-    // first factorization that needs them
-    int look = 0;            // look-ahead depth of the sweeps (with chained): 0 none, 2 or 3
-    R* l2 = nullptr;
-    R* w2 = nullptr;
-    double* bp = nullptr;
-    // the backward sweep's look-ahead system: B [nt][w] and V [nt] tiles, z' [nt * 64]
-    R* b2 = nullptr;
-    R* v2 = nullptr;
-    double* zp = nullptr;
-    // depth 3: both systems deepened by one row ([nt][w+1] tiles each) and
-    // their right-hand sides
-    R* l3 = nullptr;
-    R* b3 = nullptr;
-    double* bq = nullptr;
-    double* zq = nullptr;
+    double* bw = nullptr;
+    double* part = nullptr;
     double* xw = nullptr;    // work vectors (padded)
     double* yw = nullptr;
     int* flag = nullptr;       // error bits: 1 a wait bound hit, 2 an entry outside the band

@@ -508,13 +508,31 @@ __device__ __forceinline__ void diag_task(float (*xs)[T], float* /*ys*/, double*
 }
 
 // ---- staging ----------------------------------------------------------------
-template <bool CO, class R>
-__device__ __forceinline__ void stage(R (*dst)[T], const R* __restrict__ src) {
+template <bool CO, class D, class R>
+__device__ __forceinline__ void stage(D (*dst)[T], const R* __restrict__ src) {
     R buf[TT / NTH];   // all loads in flight before the first is used
 #pragma unroll
     for (int i = 0; i < TT / NTH; ++i) buf[i] = cld<CO>(&src[threadIdx.x + NTH * i]);
 #pragma unroll
-    for (int i = 0; i < TT / NTH; ++i) (&dst[0][0])[threadIdx.x + NTH * i] = buf[i];
+    for (int i = 0; i < TT / NTH; ++i) (&dst[0][0])[threadIdx.x + NTH * i] = D(buf[i]);
+}
+
+// dst[k][row] = src[row][k], src column-major, by 8x8 blocks: a wavefront's
+// loads touch whole 64-byte segments and its LDS writes eight rows
+template <class D, class R>
+__device__ __forceinline__ void stage_t(D (*dst)[T], const R* __restrict__ src) {
+    const int r = threadIdx.x & 7, c = threadIdx.x >> 3 & 7, wv = threadIdx.x >> 6;
+    R buf[64 / NWAVE];
+#pragma unroll
+    for (int i = 0; i < 64 / NWAVE; ++i) {
+        const int b = wv + NWAVE * i;
+        buf[i] = src[(8 * (b >> 3) + c) * T + 8 * (b & 7) + r];
+    }
+#pragma unroll
+    for (int i = 0; i < 64 / NWAVE; ++i) {
+        const int b = wv + NWAVE * i;
+        dst[8 * (b & 7) + r][8 * (b >> 3) + c] = D(buf[i]);
+    }
 }
 // A tile from LDS to memory by nthr threads, coherently, 16 bytes a store
 template <class R>
@@ -1215,532 +1233,235 @@ __global__ void __launch_bounds__(256) k_bwd_sweep(const R* __restrict__ tiles_t
     if (tid < T) put_value(&x[I * T + tid], part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid]);
 }
 
-// ---- sweeps with a precomputed chain matrix ----------------------------------
-// In the sweeps above the last step of a tile row waits for its predecessor
-// and then applies two dependent 64x64 products (L_{I,I-1} y_{I-1}, then Linv_I).
-// After each factorization k_sweep_chain forms per tile row
-//   M_I = Linv_I L_{I,I-1}            (column-major, for the forward sweep)
-//   G_I = L_{I+1,I} Linv_I            (row-major, for the backward sweep)
-// so that y_I = U_I - M_I y_{I-1}, U_I = Linv_I (b_I - sum_{J <= I-2} L_IJ y_J),
-// and x_I = U'_I - G_I^T x_{I+1}, U'_I = Linv_I^T (y_I / D_I - sum_{J >= I+2} L_JI^T x_J).
-// U_I needs the rows up to I-2 only, which arrive one chain step before
-// y_{I-1}; once y_{I-1} lands the row takes one 64x64 product and one
-// reduction.  Each workgroup still reads only its own tile row (the older
-// contributions' bandwidth per workgroup is that of the sweeps above).
-
-// tile (I, J) of the factor, I > J, read as doubles; zero outside the band
-template <class R> struct TileRd {
-    const R* p;
-    __device__ double operator()(int r, int c) const { return p ? double(p[c * T + r]) : 0.0; }
-};
-template <class R> __device__ inline TileRd<R> factor_tile(const R* tiles, long I, long J, long nt, int w) {
-    if (J < 0 || I >= nt || I - J > w || I - J < 1) return TileRd<R>{nullptr};
-    return TileRd<R>{tiles + tile_index(I, J, w) * TT};
-}
-template <class R> __device__ inline TileRd<R> linv_tile(const R* linv, long I, long nt) {
-    return TileRd<R>{(I >= 0 && I < nt) ? linv + I * TT : nullptr};
-}
-
-// acc[j] += sum_k A(r, k) B(k, c0 + j), j < 16 (B's reads are uniform over a wavefront)
-template <class FA, class FB> __device__ inline void mm64(const FA& A, const FB& B, int r, int c0, double* acc) {
-    for (int k = 0; k < T; ++k) {
-        const double a = A(r, k);
-#pragma unroll
-        for (int j = 0; j < 16; ++j) acc[j] += a * B(k, c0 + j);
-    }
-}
-
-// M_I and G_I for every tile row: one workgroup per row, thread (r, c0)
-// forming entries (r, c0..c0+15) of each product.
-template <class R>
-__global__ void __launch_bounds__(256) k_sweep_chain(const R* __restrict__ tiles, const R* __restrict__ linv,
-                                                     R* __restrict__ mch, R* __restrict__ gch, long nt, int w) {
-    const long I = blockIdx.x;
-    const int r = threadIdx.x % T, c0 = 16 * (threadIdx.x / T);
-    double acc[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[j] = 0.0;
-    mm64(linv_tile(linv, I, nt), factor_tile(tiles, I, I - 1, nt, w), r, c0, acc);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) mch[I * TT + (c0 + j) * T + r] = R(acc[j]);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[j] = 0.0;
-    mm64(factor_tile(tiles, I + 1, I, nt, w), linv_tile(linv, I, nt), r, c0, acc);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) gch[I * TT + r * T + c0 + j] = R(acc[j]);
-}
-
-// y_I = U_I - M_I y_{I-1}.  r is read from xr, whose slot I is set to SENT for
-// the backward sweep; y must hold SENT.
-template <class R>
-__global__ void __launch_bounds__(256) k_fwd_sweep_m(const R* __restrict__ tiles, const R* __restrict__ linv,
-                                                     const R* __restrict__ mch, double* __restrict__ xr, double* y,
-                                                     long nt, int w, long spin_limit, int* err) {
-    __shared__ double vin[T];
-    __shared__ double vch[NCH][T];
-    __shared__ double part[4][T];
-    const long I = blockIdx.x;
-    const int tid = threadIdx.x, row = tid % T, q = tid / T, k0 = 16 * q;
-    R lv[16], lm[16];
-    const R* lvp = linv + I * (long)TT;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) lv[k] = lvp[(k0 + k) * T + row];
-    const bool has_prev = I >= 1;
-    if (has_prev) {
-        const R* lmp = mch + I * (long)TT;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) lm[k] = lmp[(k0 + k) * T + row];
-    }
-    double acc = 0.0;
-    if (q == 0) {
-        acc = xr[I * T + row];
-        xr[I * T + row] = __builtin_bit_cast(double, SENT);
-    }
-    // the older rows J <= I - 2 in chunks of NCH, wavefront c polling row J + c
-    const long J0 = I - w > 0 ? I - w : 0;
-    for (long J = J0; J < I - 1; J += NCH) {
-        const int nc = (I - 1 - J < NCH) ? int(I - 1 - J) : NCH;
-        R lx[NCH][16];
-#pragma unroll
-        for (int c = 0; c < NCH; ++c)
-            if (c < nc) {
-                const R* l = tiles + (I * (w + 1) + (J + c - I + w)) * (long)TT;
-#pragma unroll
-                for (int k = 0; k < 16; ++k) lx[c][k] = l[(k0 + k) * T + row];
-            }
-        fetch_rows(y, J, 1, nc, vch, spin_limit, err);
-#pragma unroll
-        for (int c = 0; c < NCH; ++c)
-            if (c < nc) {
-#pragma unroll
-                for (int k = 0; k < 16; ++k) acc -= double(lx[c][k]) * vch[c][k0 + k];
-            }
-        __syncthreads();
-    }
-    // U_I = Linv_I S_I, formed before y_{I-1} is needed
-    part[q][row] = acc;
-    __syncthreads();
-    if (tid < T) vin[tid] = part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid];
-    __syncthreads();
-    double u = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) u += double(lv[k]) * vin[k0 + k];
-    __syncthreads();
-    part[q][row] = u;
-    __syncthreads();
-    double yi = (q == 0) ? part[0][row] + part[1][row] + part[2][row] + part[3][row] : 0.0;
-    if (has_prev) {
-        fetch_row(y, I - 1, vin, spin_limit, err);
-        double m = 0.0;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) m += double(lm[k]) * vin[k0 + k];
-        part[q][row] = m;
-        __syncthreads();
-        if (q == 0) yi -= part[0][row] + part[1][row] + part[2][row] + part[3][row];
-    }
-    if (q == 0) put_value(&y[I * T + row], yi);
-}
-
-// x_I = U'_I - G_I^T x_{I+1}; workgroup g handles I = nt-1-g.  x must hold SENT.
-template <class R>
-__global__ void __launch_bounds__(256) k_bwd_sweep_m(const R* __restrict__ tiles_t, const R* __restrict__ linv,
-                                                     const R* __restrict__ gch, const double* __restrict__ y,
-                                                     const double* __restrict__ piv, double* x, long nt, int w,
-                                                     long spin_limit, int* err) {
-    __shared__ double vin[T];
-    __shared__ double vch[NCH][T];
-    __shared__ double part[4][T];
-    const long I = nt - 1 - blockIdx.x;
-    const int tid = threadIdx.x, col = tid % T, q = tid / T, k0 = 16 * q;
-    R lv[16], lm[16];
-    const R* lvp = linv + I * (long)TT;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) lv[k] = lvp[col * T + k0 + k];   // Linv[k][col]
-    const bool has_next = I + 1 < nt;
-    if (has_next) {
-        const R* lgp = gch + I * (long)TT;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) lm[k] = lgp[(k0 + k) * T + col];   // G_I[k][col]
-    }
-    double acc = (q == 0) ? y[I * T + col] / piv[I * T + col] : 0.0;
-    // the later rows J >= I + 2 in chunks of NCH, wavefront c polling row J - c
-    const long J1 = (I + w < nt - 1) ? I + w : nt - 1;
-    for (long J = J1; J > I + 1; J -= NCH) {
-        const int nc = (J - (I + 1) < NCH) ? int(J - (I + 1)) : NCH;
-        R lx[NCH][16];
-#pragma unroll
-        for (int c = 0; c < NCH; ++c)
-            if (c < nc) {
-                const R* l = tiles_t + ((J - c) * (w + 1) + (I - (J - c) + w)) * (long)TT;
-#pragma unroll
-                for (int k = 0; k < 16; ++k) lx[c][k] = l[(k0 + k) * T + col];
-            }
-        fetch_rows(x, J, -1, nc, vch, spin_limit, err);
-#pragma unroll
-        for (int c = 0; c < NCH; ++c)
-            if (c < nc) {
-#pragma unroll
-                for (int k = 0; k < 16; ++k) acc -= double(lx[c][k]) * vch[c][k0 + k];
-            }
-        __syncthreads();
-    }
-    part[q][col] = acc;
-    __syncthreads();
-    if (tid < T) vin[tid] = part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid];
-    __syncthreads();
-    double u = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) u += double(lv[k]) * vin[k0 + k];
-    __syncthreads();
-    part[q][col] = u;
-    __syncthreads();
-    double xi = (q == 0) ? part[0][col] + part[1][col] + part[2][col] + part[3][col] : 0.0;
-    if (has_next) {
-        fetch_row(x, I + 1, vin, spin_limit, err);
-        double m = 0.0;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) m += double(lm[k]) * vin[k0 + k];
-        part[q][col] = m;
-        __syncthreads();
-        if (q == 0) xi -= part[0][col] + part[1][col] + part[2][col] + part[3][col];
-    }
-    if (q == 0) put_value(&x[I * T + col], xi);
-}
-
-// ---- look-ahead forward sweep -------------------------------------------------
-// Row I of the block system L y = b, multiplied by Linv_I, less W_I = M_I
-// Linv_{I-1} times row I-1 (multiplied by Linv_{I-1}), has no coupling to row
-// I-1 any more (Linv_I L_{I,I-1} - M_I = 0):
-//   y_I = b'_I - sum_{J=I-w-1}^{I-2} L'_IJ y_J,
-//   b'_I = Linv_I b_I - W_I b_{I-1},  L'_IJ = Linv_I L_IJ - W_I L_{I-1,J}.
-// The newest row a row waits for is then I-2, so the even and the odd rows
-// form two chains that run side by side.  L' is kept per row in w slots, slot
-// s for J = I-2-s (column-major tiles), formed after each factorization.
-
-// W_I = M_I Linv_{I-1} (I >= 1), column-major.  Y^T = Linv_{I-1}: ys[k][col] =
-// Linv_{I-1}[k][col], a transposed staging of the column-major tile.
-template <class R>
-__global__ void __launch_bounds__(NTH) k_look2_w(const R* __restrict__ mch, const R* __restrict__ linv,
-                                                 R* __restrict__ w2, long nt) {
-    __shared__ R xs[T][T];
-    __shared__ R ys[T][T];
-    const long I = blockIdx.x + 1;
-    stage<false>(xs, mch + I * (long)TT);
-    const R* lv = linv + (I - 1) * (long)TT;
-    for (int idx = threadIdx.x; idx < TT; idx += NTH) ys[idx % T][idx / T] = lv[idx];
-    __syncthreads();
-    TileAcc<R> acc;
-    acc.product(xs, ys);
-    acc.each([&](int row, int col, R v) { w2[I * (long)TT + col * T + row] = v; });
-}
-
-// L'_{I, I-2-s} for workgroup (I, s): Linv_I L_IJ (when I - J <= w) less
-// W_I L_{I-1,J}; the L tiles are staged from their row-major transposed
-// copies, so that ys[k][col] = L[k][col] reads straight.
-template <class R>
-__global__ void __launch_bounds__(NTH) k_look2_band(const R* __restrict__ tiles_t, const R* __restrict__ linv,
-                                                    const R* __restrict__ w2, R* __restrict__ l2, long nt, int w) {
-    __shared__ R xs[T][T];
-    __shared__ R ys[T][T];
-    const long I = blockIdx.x / w;
-    const int s = int(blockIdx.x % w);
-    const long J = I - 2 - s;
-    if (J < 0) return;
-    TileAcc<R> a, b;
-    const bool direct = I - J <= w;
-    if (direct) {
-        stage<false>(xs, linv + I * (long)TT);
-        stage<false>(ys, tiles_t + tile_index(I, J, w) * TT);
-        __syncthreads();
-        a.product(xs, ys);
-        __syncthreads();
-    }
-    stage<false>(xs, w2 + I * (long)TT);
-    stage<false>(ys, tiles_t + tile_index(I - 1, J, w) * TT);
-    __syncthreads();
-    b.product(xs, ys);
-    R* out = l2 + (I * w + s) * (long)TT;
-    if (direct) {
-        R av[TileAcc<R>::N];
-        a.each_i([&](int, int, R v, int e) { av[e] = v; });
-        b.each_i([&](int row, int col, R v, int e) { out[col * T + row] = av[e] - v; });
-    } else {
-        b.each([&](int row, int col, R v) { out[col * T + row] = -v; });
-    }
-}
-
-// b'_I = Linv_I b_I - W_I b_{I-1}, one workgroup per tile row, thread (row, q)
-// summing columns 16q..16q+15
-template <class R>
-__global__ void __launch_bounds__(256) k_look2_rhs(const R* __restrict__ linv, const R* __restrict__ w2,
-                                                   const double* __restrict__ b, double* __restrict__ bp, long nt) {
-    __shared__ double part[4][T];
-    const long I = blockIdx.x;
-    const int tid = threadIdx.x, row = tid % T, q = tid / T, k0 = 16 * q;
-    const R* lv = linv + I * (long)TT;
-    double u = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) u += double(lv[(k0 + k) * T + row]) * b[I * T + k0 + k];
-    if (I >= 1) {
-        const R* wv = w2 + I * (long)TT;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) u -= double(wv[(k0 + k) * T + row]) * b[(I - 1) * T + k0 + k];
-    }
-    part[q][row] = u;
-    __syncthreads();
-    if (tid < T) bp[I * T + tid] = part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid];
-}
-
-// The look-ahead sweeps take their older rows NCW at a time: a workgroup
-// catching up behind the front consumes one chunk per memory round trip, so
-// the front advances at most NCW rows per round trip whatever the depth of
-// the system.  Eight waves, thread (row, q) holding columns 8q..8q+7 of each
-// tile; a chunk's tile loads are issued before its rows are polled and share
-// that round trip.
-constexpr int NCW = 8;
+// ---- block sweeps --------------------------------------------------------------
+// Above, every tile row waits for the one before: about 1 us a row of store,
+// poll and products, however fast the tiles stream.  The default schedule
+// takes SB tile rows at a time.  With Linv_B the inverse of a block's SB x SB
+// tiles of L, formed after each factorization,
+//   y_B = Linv_B S_B - M_B y_{B-1},  S_B = b_B - sum over the rows before block B-1,
+//   M_B = Linv_B L_{B,B-1},
+// so a block waits once for its predecessor, and everything else of it is
+// formed meanwhile.  The backward sweep is the same on L^T: x_B = Linv_B^T S'_B -
+// G_B x_{B+1}, G_B = Linv_B^T L_{B+1,B}^T, S'_B = y_B / D_B - sum over the rows past
+// block B+1.
+// The products of a block are spread over many workgroups, which load their
+// tiles into registers before they wait: a sweep has few rows in progress
+// at once, and one workgroup per row could not stream a row's tiles in the
+// time the front takes to pass it.  A block has 4 (gh + 1) workgroups of 512
+// threads: for each row gh helpers, each with up to HT tiles of the older
+// rows, which leave partial sums, and one that finishes the row.
+// 256 x 256 panel (6168 rows, 25 tiles below the diagonal): 2.44 / 2.50 ms
+// forward / backward (2.5 TB/s of 6.0 GB) and 2.7 ms to form the matrices per
+// factorization; one row at a time took 6.2 / 6.5 ms, and systems that
+// decoupled each row from the one or two before 5.1 / 5.2 ms with 11 ms of
+// forming.  A band of a single block has nothing to overlap and takes the
+// row sweeps, which need nothing formed (BandLDLT::blocked).
+constexpr int SB = 4;      // tile rows per block
+constexpr int HT = 8;      // tiles per helper; a wavefront polls one of their rows
 constexpr int SWT = 512;
+constexpr int LB = SB * (SB - 1) / 2;   // off-diagonal tiles of Linv_B
+__device__ __forceinline__ long lb_index(long b, int i, int k) { return (b * LB + i * (i - 1) / 2 + k) * TT; }   // i > k
 
-// y_I = b'_I - sum_{J=I-w-D+1}^{I-D} L'_IJ y_J on a look-ahead system of
-// depth D (slot s of row I for J = I-D-s, w slots), the older rows in chunks
-// of NCW aligned so that the last chunk ends at row I-D: a row waits once for
-// the newest rows it needs and the D chains of the system (the rows of each
-// residue mod D) run side by side.  y must hold SENT.
+// Linv_B below its diagonal tiles, column by column: workgroup (b, j) forms
+// Linv_ij = -Linv_i sum_{k=j}^{i-1} L_ik Linv_kj for i = j+1 .. (FP64 products)
 template <class R>
-__global__ void __launch_bounds__(SWT) k_fwd_sweep_la(const R* __restrict__ l2, const double* __restrict__ bp,
-                                                      double* y, long nt, int w, int D, long spin_limit, int* err) {
-    __shared__ double vch[NCW][T];
-    __shared__ double part[SWT / T][T];
-    const long I = blockIdx.x;
-    const int tid = threadIdx.x, row = tid % T, q = tid / T, k0 = 8 * q;
-    double acc = (q == 0) ? bp[I * T + row] : 0.0;
-    const long J0 = I - w - D + 1 > 0 ? I - w - D + 1 : 0;
-    const long nrow = I - D + 1 - J0;   // rows J0 .. I-D
-    int nc = int(nrow % NCW);
-    if (nc == 0) nc = NCW;
-    for (long J = J0; J <= I - D; J += nc, nc = NCW) {
-        R lx[NCW][8];
-#pragma unroll
-        for (int c = 0; c < NCW; ++c)
-            if (c < nc) {
-                const R* l = l2 + (I * w + (I - D - (J + c))) * (long)TT;
-#pragma unroll
-                for (int k = 0; k < 8; ++k) lx[c][k] = l[(k0 + k) * T + row];
-            }
-        fetch_rows(y, J, 1, nc, vch, spin_limit, err);
-#pragma unroll
-        for (int c = 0; c < NCW; ++c)
-            if (c < nc) {
-#pragma unroll
-                for (int k = 0; k < 8; ++k) acc -= double(lx[c][k]) * vch[c][k0 + k];
-            }
-        __syncthreads();
-    }
-    part[q][row] = acc;
-    __syncthreads();
-    if (q == 0) {
-        double v = part[0][row];
-#pragma unroll
-        for (int g = 1; g < SWT / T; ++g) v += part[g][row];
-        put_value(&y[I * T + row], v);
-    }
-}
-
-// The backward sweep x_I = Linv_I^T (z_I - sum_{J>I} L_JI^T x_J), z = y / d,
-// on the same look-ahead system: with V_I = G_I^T Linv_{I+1}^T the coupling
-// to x_{I+1} cancels and
-//   x_I = z'_I - sum_{J=I+2}^{I+w+1} B_IJ x_J,
-//   z'_I = Linv_I^T z_I - V_I z_{I+1},  B_IJ = Linv_I^T L_JI^T - V_I L_{J,I+1}^T,
-// B kept per row in w slots, slot s for J = I+2+s (column-major tiles).
-
-// V_I (I <= nt-2): X = G_I^T (G_I row-major: xs[k][row] = G_I[k][row]),
-// Y = Linv_{I+1} (ys[k][col] = Linv_{I+1}[col][k], column-major storage)
-template <class R>
-__global__ void __launch_bounds__(NTH) k_look2_v(const R* __restrict__ gch, const R* __restrict__ linv,
-                                                 R* __restrict__ v2, long nt) {
-    __shared__ R xs[T][T];
-    __shared__ R ys[T][T];
-    const long I = blockIdx.x;
-    stage<false>(xs, gch + I * (long)TT);
-    stage<false>(ys, linv + (I + 1) * (long)TT);
-    __syncthreads();
-    TileAcc<R> acc;
-    acc.product(xs, ys);
-    acc.each([&](int row, int col, R v) { v2[I * (long)TT + col * T + row] = v; });
-}
-
-// B_{I, I+2+s} for workgroup (I, s): X = Linv_I^T (a transposed staging of the
-// column-major tile) with Y = L_JI, less X = V_I with Y = L_{J,I+1}; the L
-// tiles are column-major, so ys[k][col] = L[col][k] stages straight.
-template <class R>
-__global__ void __launch_bounds__(NTH) k_look2_bband(const R* __restrict__ tiles, const R* __restrict__ linv,
-                                                     const R* __restrict__ v2, R* __restrict__ b2, long nt,
-                                                     int w) {
-    __shared__ R xs[T][T];
-    __shared__ R ys[T][T];
-    const long I = blockIdx.x / w;
-    const int s = int(blockIdx.x % w);
-    const long J = I + 2 + s;
-    if (J >= nt) return;
-    TileAcc<R> a, b;
-    const bool direct = J - I <= w;
-    if (direct) {
-        const R* lv = linv + I * (long)TT;
-        for (int idx = threadIdx.x; idx < TT; idx += NTH) xs[idx % T][idx / T] = lv[idx];
-        stage<false>(ys, tiles + tile_index(J, I, w) * TT);
-        __syncthreads();
-        a.product(xs, ys);
-        __syncthreads();
-    }
-    stage<false>(xs, v2 + I * (long)TT);
-    stage<false>(ys, tiles + tile_index(J, I + 1, w) * TT);
-    __syncthreads();
-    b.product(xs, ys);
-    R* out = b2 + (I * w + s) * (long)TT;
-    if (direct) {
-        R av[TileAcc<R>::N];
-        a.each_i([&](int, int, R v, int e) { av[e] = v; });
-        b.each_i([&](int row, int col, R v, int e) { out[col * T + row] = av[e] - v; });
-    } else {
-        b.each([&](int row, int col, R v) { out[col * T + row] = -v; });
-    }
-}
-
-// z'_I = Linv_I^T z_I - V_I z_{I+1}, z = y / d, one workgroup per tile row
-template <class R>
-__global__ void __launch_bounds__(256) k_look2_brhs(const R* __restrict__ linv, const R* __restrict__ v2,
-                                                    const double* __restrict__ y, const double* __restrict__ piv,
-                                                    double* __restrict__ zp, long nt) {
-    __shared__ double part[4][T];
-    const long I = blockIdx.x;
-    const int tid = threadIdx.x, row = tid % T, q = tid / T, k0 = 16 * q;
-    const R* lv = linv + I * (long)TT;
-    double u = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const long e = I * T + k0 + k;
-        u += double(lv[row * T + k0 + k]) * (y[e] / piv[e]);   // Linv_I[k][row]
-    }
-    if (I + 1 < nt) {
-        const R* vv = v2 + I * (long)TT;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const long e = (I + 1) * T + k0 + k;
-            u -= double(vv[(k0 + k) * T + row]) * (y[e] / piv[e]);
+__global__ void __launch_bounds__(NTH) k_block_inverse(const R* __restrict__ tiles, const R* __restrict__ linv,
+                                                       R* __restrict__ lb, long nt, int w) {
+    __shared__ double xs[T][T], ys[T][T];
+    __shared__ double vs[SB - 2][T][T];   // Linv_kj, k > j, row-major
+    const long b = blockIdx.x / (SB - 1);
+    const int j = int(blockIdx.x % (SB - 1)), nr = int(min(long(SB), nt - SB * b));
+    for (int i = j + 1; i < nr; ++i) {
+        const long I = SB * b + i;
+        double sum[TileAcc<double>::N] = {};
+        TileAcc<double> acc;
+        for (int k = j; k < i; ++k) {
+            if (i - k > w) continue;
+            stage<false>(xs, tiles + tile_index(I, SB * b + k, w) * TT);
+            if (k == j) stage_t(ys, linv + (SB * b + j) * (long)TT);
+            __syncthreads();
+            acc.product(xs, k == j ? ys : vs[k - j - 1]);
+            acc.each_i([&](int, int, double v, int e) { sum[e] += v; });
+            __syncthreads();
         }
+        stage<false>(xs, linv + I * (long)TT);
+        acc.each_i([&](int row, int col, double, int e) { ys[row][col] = sum[e]; });
+        __syncthreads();
+        acc.product(xs, ys);
+        R* out = lb + lb_index(b, i, j);
+        acc.each([&](int row, int col, double v) {
+            out[col * T + row] = R(-v);
+            if (i - j - 1 < SB - 2) vs[i - j - 1][row][col] = -v;
+        });
+        __syncthreads();
     }
-    part[q][row] = u;
-    __syncthreads();
-    if (tid < T) zp[I * T + tid] = part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid];
 }
 
-// x_I = z'_I - sum_{J=I+D}^{I+D+w-1} B_IJ x_J on a look-ahead system of depth
-// D (slot s of row I for J = I+D+s), I = nt-1-blockIdx.x: the later rows in
-// chunks of NCW, farthest first, aligned so that the last chunk ends at row
-// I+D.  x must hold SENT.
+// Whether M_B (dir 1) or G_B (dir -1) has a tile in column j of its block: the
+// row or column of the band nearest to it reaches it.
+__device__ __forceinline__ bool has_link(bool fwd, long b, int j, long nt, int w) {
+    return fwd ? b >= 1 && SB - j <= w : SB * (b + 1) + j < nt && j < w;
+}
+
+// Tile (i, j) of M_B (the first half of the grid) or of G_B (the second),
+// column-major, at [SB b + i][j]
 template <class R>
-__global__ void __launch_bounds__(SWT) k_bwd_sweep_la(const R* __restrict__ b2, const double* __restrict__ zp,
-                                                      double* x, long nt, int w, int D, long spin_limit, int* err) {
-    __shared__ double vch[NCW][T];
-    __shared__ double part[SWT / T][T];
-    const long I = nt - 1 - blockIdx.x;
-    const int tid = threadIdx.x, row = tid % T, q = tid / T, k0 = 8 * q;
-    double acc = (q == 0) ? zp[I * T + row] : 0.0;
-    const long J1 = (I + D + w - 1 < nt - 1) ? I + D + w - 1 : nt - 1;
-    const long nrow = J1 - (I + D) + 1;   // rows J1 down to I+D
-    int nc = int(nrow % NCW);
-    if (nc == 0) nc = NCW;
-    for (long J = J1; J >= I + D; J -= nc, nc = NCW) {
-        R lx[NCW][8];
+__global__ void __launch_bounds__(NTH) k_block_link(const R* __restrict__ tiles, const R* __restrict__ tiles_t,
+                                                    const R* __restrict__ linv, const R* __restrict__ lb,
+                                                    R* __restrict__ mch, R* __restrict__ gch, long nt, int w) {
+    __shared__ double xs[T][T], ys[T][T];
+    const bool fwd = blockIdx.x < nt * SB;
+    const long q = fwd ? blockIdx.x : blockIdx.x - nt * SB, I = q / SB, b = I / SB;
+    const int i = int(I % SB), j = int(q % SB);
+    if (!has_link(fwd, b, j, nt, w)) return;
+    double sum[TileAcc<double>::N] = {};
+    TileAcc<double> acc;
+    for (int k = fwd ? 0 : i; k <= (fwd ? i : SB - 1); ++k) {
+        const long K = SB * b + k;
+        if ((fwd ? SB + k - j : SB + j - k) > w) continue;
+        if (fwd) {
+            stage<false>(xs, k == i ? linv + I * (long)TT : lb + lb_index(b, i, k));
+            stage<false>(ys, tiles_t + tile_index(K, SB * (b - 1) + j, w) * TT);
+        } else {
+            stage_t(xs, k == i ? linv + I * (long)TT : lb + lb_index(b, k, i));
+            stage<false>(ys, tiles + tile_index(SB * (b + 1) + j, K, w) * TT);
+        }
+        __syncthreads();
+        acc.product(xs, ys);
+        acc.each_i([&](int, int, double v, int e) { sum[e] += v; });
+        __syncthreads();
+    }
+    R* out = (fwd ? mch : gch) + q * (long)TT;
+    acc.each_i([&](int row, int col, double, int e) { out[col * T + row] = R(sum[e]); });
+}
+
+inline int helpers_per_row(int w) { return std::max(0, (w - SB + HT - 1) / HT); }
+
+// One sweep: v = the solution, every slot SENT before; part [nt][gh][T], SENT.
+// FWD: v = y from rhs = b.  Otherwise v = x from rhs = y and the pivots, with
+// the transposed tiles.  Workgroups in the order of the blocks, a block's
+// helpers (oldest rows first) before its finishing workgroups, so that each
+// waits on lower ones only.
+template <class R, bool FWD>
+__global__ void __launch_bounds__(SWT) k_sweep_block(const R* __restrict__ tl, const R* __restrict__ linv,
+                                                     const R* __restrict__ lb, const R* __restrict__ link,
+                                                     const double* __restrict__ rhs, const double* __restrict__ piv,
+                                                     double* v, double* part, long nt, int w, int gh, long spin_limit,
+                                                     int* err) {
+    __shared__ double vch[HT][T];
+    __shared__ double red[SWT / T][T];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, k0 = 8 * wv;
+    const long nb = (nt + SB - 1) / SB, per = SB * (gh + 1);
+    const long b = FWD ? blockIdx.x / per : nb - 1 - blockIdx.x / per;
+    const int r = int(blockIdx.x % per), i = r % SB;
+    const long I = SB * b + i;
+    if (I >= nt) return;
+    // older rows of row I by groups of HT, group 0 the newest: first and last
+    // row (towards older rows) of group g, none left when the count is <= 0
+    const int dir = FWD ? -1 : 1;
+    auto group = [&](long row, int g, long& first) {
+        first = FWD ? SB * (b - 1) - 1 - HT * g : SB * (b + 2) + HT * g;
+        const long last = FWD ? max(0L, row - w) : min(nt - 1, row + w);
+        return int(min(long(HT), FWD ? first - last + 1 : last - first + 1));
+    };
+    auto finish = [&](double acc, double* out) {
+        red[wv][lane] = acc;
+        __syncthreads();
+        if (wv == 0) {
+            double s = red[0][lane];
 #pragma unroll
-        for (int c = 0; c < NCW; ++c)
-            if (c < nc) {
-                const R* l = b2 + (I * w + (J - c - I - D)) * (long)TT;
+            for (int q = 1; q < SWT / T; ++q) s += red[q][lane];
+            put_value(out, s);
+        }
+    };
+    if (r < SB * gh) {
+        const int g = gh - 1 - r / SB;
+        long first;
+        const int n = group(I, g, first);
+        if (n <= 0) return;
+        R lx[HT][8];
 #pragma unroll
-                for (int k = 0; k < 8; ++k) lx[c][k] = l[(k0 + k) * T + row];
+        for (int c = 0; c < HT; ++c)
+            if (c < n) {
+                const long J = first + dir * c;
+                const R* l = tl + (FWD ? tile_index(I, J, w) : tile_index(J, I, w)) * TT;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) lx[c][k] = l[(k0 + k) * T + lane];
             }
-        fetch_rows(x, J, -1, nc, vch, spin_limit, err);
+        if (wv < n) vch[wv][lane] = poll_value(v + (first + dir * wv) * T + lane, spin_limit, err);
+        __syncthreads();
+        double acc = 0.0;
 #pragma unroll
-        for (int c = 0; c < NCW; ++c)
-            if (c < nc) {
+        for (int c = 0; c < HT; ++c)
+            if (c < n) {
 #pragma unroll
                 for (int k = 0; k < 8; ++k) acc -= double(lx[c][k]) * vch[c][k0 + k];
             }
-        __syncthreads();
-    }
-    part[q][row] = acc;
-    __syncthreads();
-    if (q == 0) {
-        double v = part[0][row];
-#pragma unroll
-        for (int g = 1; g < SWT / T; ++g) v += part[g][row];
-        put_value(&x[I * T + row], v);
-    }
-}
-
-// ---- deeper look-ahead -------------------------------------------------------
-// A look-ahead system of depth D (row I coupled to row I-D and rows further
-// back, slot s of row I holding the tile for J = I-D-s, ws slots) is deepened
-// by substituting row I-D's own equation for the coupling P_I (slot 0) to it:
-//   L+_IJ = L_IJ - P_I L_{I-D,J},  b+_I = b_I - P_I b_{I-D},
-// which couples row I to rows I-D-1 and further back in ws + D - 1 slots: slot
-// s (J = I-D-1-s) is slot s+1 of row I less P_I times slot s+1-D of row I-D.
-// The backward system deepens the same way towards the later rows (J =
-// I+D+1+s, row I+D): dir = +1 forward, -1 backward.  Every slot whose row J
-// exists is written (zero where neither term has a tile).
-template <class R>
-__global__ void __launch_bounds__(NTH) k_look_deepen(const R* __restrict__ src, int ws, R* __restrict__ dst, int wd,
-                                                     long nt, int D, int dir) {
-    __shared__ R xs[T][T];
-    __shared__ R ys[T][T];
-    const long I = blockIdx.x / wd;
-    const int s = int(blockIdx.x % wd);
-    const long J = I - long(dir) * (D + 1 + s);
-    if (J < 0 || J >= nt) return;
-    R* out = dst + (I * wd + s) * (long)TT;
-    const R* keep = (s + 1 <= ws - 1) ? src + (I * ws + s + 1) * (long)TT : nullptr;
-    const int sr = s + 1 - D;   // <= ws - 1 for every s < wd
-    if (sr < 0) {
-        for (int idx = threadIdx.x; idx < TT; idx += NTH) out[idx] = keep ? keep[idx] : R(0);
+        finish(acc, &part[(I * gh + g) * T + lane]);
         return;
     }
-    const long Ir = I - long(dir) * D;
-    stage<false>(xs, src + I * ws * (long)TT);   // P_I, column-major: xs[k][row] = P_I[row][k]
-    const R* y = src + (Ir * ws + sr) * (long)TT;
-    for (int idx = threadIdx.x; idx < TT; idx += NTH) ys[idx % T][idx / T] = y[idx];
-    __syncthreads();
-    TileAcc<R> acc;
-    acc.product(xs, ys);
-    if (keep)
-        acc.each([&](int row, int col, R v) { out[col * T + row] = keep[col * T + row] - v; });
-    else
-        acc.each([&](int row, int col, R v) { out[col * T + row] = -v; });
-}
-
-// b+_I = b_I - P_I b_{I-dir*D} with P_I slot 0 of row I of the depth-D
-// system, one workgroup per tile row
-template <class R>
-__global__ void __launch_bounds__(256) k_look_deepen_rhs(const R* __restrict__ src, int ws,
-                                                         const double* __restrict__ b, double* __restrict__ bo,
-                                                         long nt, int D, int dir) {
-    __shared__ double part[4][T];
-    const long I = blockIdx.x;
-    const int tid = threadIdx.x, row = tid % T, q = tid / T, k0 = 16 * q;
-    const long Ir = I - long(dir) * D;
-    double u = (q == 0) ? b[I * T + row] : 0.0;
-    if (Ir >= 0 && Ir < nt) {
-        const R* pv = src + I * ws * (long)TT;
+    const int nr = int(min(long(SB), nt - SB * b));
+    R li[SB][8], lm[SB][8];
+    bool linked[SB];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) u -= double(pv[(k0 + k) * T + row]) * b[Ir * T + k0 + k];
+    for (int k = 0; k < SB; ++k) {
+        linked[k] = has_link(FWD, b, k, nt, w);
+        if (linked[k]) {
+            const R* l = link + (I * SB + k) * (long)TT;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) lm[k][e] = l[(k0 + e) * T + lane];
+        }
+        if (FWD ? k <= i : k >= i && k < nr) {
+            const R* l = k == i ? linv + I * (long)TT : lb + (FWD ? lb_index(b, i, k) : lb_index(b, k, i));
+#pragma unroll
+            for (int e = 0; e < 8; ++e) li[k][e] = FWD ? l[(k0 + e) * T + lane] : l[lane * T + k0 + e];
+        }
     }
-    part[q][row] = u;
+    // S of the block's rows that row I needs, a wavefront each
+    if (wv < SB && (FWD ? wv <= i : wv >= i && wv < nr)) {
+        const long K = SB * b + wv, e = K * T + lane;
+        double s = FWD ? rhs[e] : rhs[e] / piv[e];
+        for (int g = gh - 1; g >= 0; --g) {
+            long first;
+            if (group(K, g, first) > 0) s += poll_value(&part[(K * gh + g) * T + lane], spin_limit, err);
+        }
+        vch[wv][lane] = s;
+    }
     __syncthreads();
-    if (tid < T) bo[I * T + tid] = part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid];
+    double acc = 0.0;
+#pragma unroll
+    for (int k = 0; k < SB; ++k)
+        if (FWD ? k <= i : k >= i && k < nr) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc += double(li[k][e]) * vch[k][k0 + e];
+        }
+    if (wv >= SB) {   // the neighbouring block's rows
+        const int k = wv - SB;
+        if (has_link(FWD, b, k, nt, w))
+            vch[wv][lane] = poll_value(v + ((FWD ? SB * (b - 1) : SB * (b + 1)) + k) * T + lane, spin_limit, err);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < SB; ++k)
+        if (linked[k]) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc -= double(lm[k][e]) * vch[SB + k][k0 + e];
+        }
+    finish(acc, &v[I * T + lane]);
 }
 
-// v = SENT
-__global__ void k_fill_sent(double* __restrict__ v, long n) {
-    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (i < n) v[i] = __builtin_bit_cast(double, SENT);
+// dst = rhs padded with zeros to ntot; y, x and the partial sums SENT
+__global__ void k_sweep_block_prep(double* __restrict__ dst, const double* __restrict__ src, double* __restrict__ y,
+                                   double* __restrict__ x, double* __restrict__ part, long n, long ntot, long npart) {
+    const double sent = __builtin_bit_cast(double, SENT);
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < max(ntot, npart); i += (long)gridDim.x * blockDim.x) {
+        if (i < ntot) {
+            dst[i] = i < n ? src[i] : 0.0;
+            y[i] = sent;
+            x[i] = sent;
+        }
+        if (i < npart) part[i] = sent;
+    }
 }
 
 // dst = rhs padded with zeros to ntot; y = SENT
@@ -2186,8 +1907,6 @@ void BandLDLT<R>::setup(long n_, long bandwidth, hipStream_t s_) {
     tiles = dalloc<R>(size_t(nt) * size_t(w + 1) * TT);
     tiles_t = dalloc<R>(size_t(nt) * size_t(w + 1) * TT);
     linv = dalloc<R>(size_t(nt) * TT);
-    mch = dalloc<R>(size_t(nt) * TT);
-    gch = dalloc<R>(size_t(nt) * TT);
     piv = dalloc<double>(size_t(nt) * T);
     xw = dalloc<double>(size_t(nt) * T);
     yw = dalloc<double>(size_t(nt) * T);
@@ -2200,14 +1919,11 @@ void BandLDLT<R>::setup(long n_, long bandwidth, hipStream_t s_) {
 
 template <class R>
 void BandLDLT<R>::release() {
-    void* ps[] = {tiles, tiles_t, linv, mch, gch, piv, xw, yw, flag, prog, l2, w2, bp, b2, v2, zp, l3, b3, bq, zq};
+    void* ps[] = {tiles, tiles_t, linv, lb, mch, gch, piv, xw, yw, bw, part, flag, prog};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     tiles = nullptr; tiles_t = nullptr; linv = nullptr; piv = nullptr; xw = nullptr; yw = nullptr; flag = nullptr;
-    mch = nullptr; gch = nullptr;
-    l2 = nullptr; w2 = nullptr; bp = nullptr;
-    b2 = nullptr; v2 = nullptr; zp = nullptr;
-    l3 = nullptr; b3 = nullptr; bq = nullptr; zq = nullptr;
+    lb = nullptr; mch = nullptr; gch = nullptr; bw = nullptr; part = nullptr;
     prog = nullptr;
     clock.release();
 }
@@ -2260,36 +1976,21 @@ int BandLDLT<R>::factor(const Dev& d) {
         }
     }
     CB_CHECK(hipGetLastError());
-    if (chained) {
+    if (blocked()) {
         const bool tk_prep = clock.take(KT_PREP);
         if (tk_prep) clock.begin(KT_PREP, s);
-        hipLaunchKernelGGL((k_sweep_chain<R>), dim3(int(nt)), dim3(256), 0, s, tiles, linv, mch, gch, nt, w);
-        if (look >= 2 && nt >= 2) {
-            if (!l2) {
-                l2 = dalloc<R>(size_t(nt) * size_t(w) * TT);
-                w2 = dalloc<R>(size_t(nt) * TT);
-                bp = dalloc<double>(size_t(nt) * T);
-                b2 = dalloc<R>(size_t(nt) * size_t(w) * TT);
-                v2 = dalloc<R>(size_t(nt) * TT);
-                zp = dalloc<double>(size_t(nt) * T);
-            }
-            hipLaunchKernelGGL((k_look2_w<R>), dim3(int(nt - 1)), dim3(NTH), 0, s, mch, linv, w2, nt);
-            hipLaunchKernelGGL((k_look2_band<R>), dim3(int(nt * w)), dim3(NTH), 0, s, tiles_t, linv, w2, l2, nt, w);
-            hipLaunchKernelGGL((k_look2_v<R>), dim3(int(nt - 1)), dim3(NTH), 0, s, gch, linv, v2, nt);
-            hipLaunchKernelGGL((k_look2_bband<R>), dim3(int(nt * w)), dim3(NTH), 0, s, tiles, linv, v2, b2, nt, w);
-            if (look >= 3) {
-                if (!l3) {
-                    l3 = dalloc<R>(size_t(nt) * size_t(w + 1) * TT);
-                    b3 = dalloc<R>(size_t(nt) * size_t(w + 1) * TT);
-                    bq = dalloc<double>(size_t(nt) * T);
-                    zq = dalloc<double>(size_t(nt) * T);
-                }
-                hipLaunchKernelGGL((k_look_deepen<R>), dim3(int(nt * (w + 1))), dim3(NTH), 0, s, l2, w, l3, w + 1,
-                                   nt, 2, 1);
-                hipLaunchKernelGGL((k_look_deepen<R>), dim3(int(nt * (w + 1))), dim3(NTH), 0, s, b2, w, b3, w + 1,
-                                   nt, 2, -1);
-            }
+        const long nb = (nt + SB - 1) / SB;
+        if (!lb) {
+            lb = dalloc<R>(size_t(nb) * LB * TT);
+            mch = dalloc<R>(size_t(nt) * SB * TT);
+            gch = dalloc<R>(size_t(nt) * SB * TT);
+            bw = dalloc<double>(size_t(nt) * T);
+            part = dalloc<double>(size_t(2 * nt * helpers_per_row(w) * T));
         }
+        hipLaunchKernelGGL((k_block_inverse<R>), dim3(unsigned(nb * (SB - 1))), dim3(NTH), 0, s, tiles, linv, lb, nt,
+                           w);
+        hipLaunchKernelGGL((k_block_link<R>), dim3(unsigned(2 * nt * SB)), dim3(NTH), 0, s, tiles, tiles_t, linv, lb,
+                           mch, gch, nt, w);
         if (tk_prep) clock.end(s);
         CB_CHECK(hipGetLastError());
     }
@@ -2308,46 +2009,29 @@ int BandLDLT<R>::factor(const Dev& d) {
 template <class R>
 void BandLDLT<R>::solve(const double* rhs, double* out) {
     CB_CHECK(hipMemsetAsync(flag, 0, sizeof(int), s));
-    hipLaunchKernelGGL(k_sweep_prep, dim3(int((nt * T + 255) / 256)), dim3(256), 0, s, xw, rhs, yw, n, nt * T);
-    const long spin_limit = 1L << 22;
-    const bool ahead = chained && look >= 2 && l2;
-    const bool deep = ahead && look >= 3 && l3;
-    if (ahead) {
-        hipLaunchKernelGGL((k_look2_rhs<R>), dim3(int(nt)), dim3(256), 0, s, linv, w2, xw, bp, nt);
-        if (deep)
-            hipLaunchKernelGGL((k_look_deepen_rhs<R>), dim3(int(nt)), dim3(256), 0, s, l2, w, bp, bq, nt, 2, 1);
-        hipLaunchKernelGGL(k_fill_sent, dim3(int((nt * T + 255) / 256)), dim3(256), 0, s, xw, nt * T);
-    }
+    const long spin_limit = 1L << 22, ntot = nt * T;
+    const int gh = helpers_per_row(w);
+    const long npart = nt * gh * T;
+    const unsigned grid = unsigned((nt + SB - 1) / SB * SB * (gh + 1));
+    if (blocked())
+        hipLaunchKernelGGL(k_sweep_block_prep, dim3(int(std::min(2048L, (std::max(ntot, 2 * npart) + 255) / 256))),
+                           dim3(256), 0, s, bw, rhs, yw, xw, part, n, ntot, 2 * npart);
+    else
+        hipLaunchKernelGGL(k_sweep_prep, dim3(int((ntot + 255) / 256)), dim3(256), 0, s, xw, rhs, yw, n, ntot);
     const bool tk_fwd = clock.take(KT_FWD);
     if (tk_fwd) clock.begin(KT_FWD, s);
-    if (deep)
-        hipLaunchKernelGGL((k_fwd_sweep_la<R>), dim3(int(nt)), dim3(SWT), 0, s, l3, bq, yw, nt, w + 1, 3, spin_limit,
-                           flag);
-    else if (ahead)
-        hipLaunchKernelGGL((k_fwd_sweep_la<R>), dim3(int(nt)), dim3(SWT), 0, s, l2, bp, yw, nt, w, 2, spin_limit,
-                           flag);
-    else if (chained)
-        hipLaunchKernelGGL((k_fwd_sweep_m<R>), dim3(int(nt)), dim3(256), 0, s, tiles, linv, mch, xw, yw, nt, w,
-                           spin_limit, flag);
+    if (blocked())
+        hipLaunchKernelGGL((k_sweep_block<R, true>), dim3(grid), dim3(SWT), 0, s, tiles, linv, lb, mch, bw, piv, yw,
+                           part, nt, w, gh, spin_limit, flag);
     else
         hipLaunchKernelGGL((k_fwd_sweep<R>), dim3(int(nt)), dim3(256), 0, s, tiles, linv, xw, yw, nt, w, spin_limit,
                            flag);
     if (tk_fwd) clock.end(s);
-    if (ahead)
-        hipLaunchKernelGGL((k_look2_brhs<R>), dim3(int(nt)), dim3(256), 0, s, linv, v2, yw, piv, zp, nt);
-    if (deep)
-        hipLaunchKernelGGL((k_look_deepen_rhs<R>), dim3(int(nt)), dim3(256), 0, s, b2, w, zp, zq, nt, 2, -1);
     const bool tk_bwd = clock.take(KT_BWD);
     if (tk_bwd) clock.begin(KT_BWD, s);
-    if (deep)
-        hipLaunchKernelGGL((k_bwd_sweep_la<R>), dim3(int(nt)), dim3(SWT), 0, s, b3, zq, xw, nt, w + 1, 3, spin_limit,
-                           flag);
-    else if (ahead)
-        hipLaunchKernelGGL((k_bwd_sweep_la<R>), dim3(int(nt)), dim3(SWT), 0, s, b2, zp, xw, nt, w, 2, spin_limit,
-                           flag);
-    else if (chained)
-        hipLaunchKernelGGL((k_bwd_sweep_m<R>), dim3(int(nt)), dim3(256), 0, s, tiles_t, linv, gch, yw, piv, xw, nt, w,
-                           spin_limit, flag);
+    if (blocked())
+        hipLaunchKernelGGL((k_sweep_block<R, false>), dim3(grid), dim3(SWT), 0, s, tiles_t, linv, lb, gch, yw, piv, xw,
+                           part + npart, nt, w, gh, spin_limit, flag);
     else
         hipLaunchKernelGGL((k_bwd_sweep<R>), dim3(int(nt)), dim3(256), 0, s, tiles_t, linv, yw, piv, xw, nt, w,
                            spin_limit, flag);

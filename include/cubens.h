@@ -95,15 +95,12 @@ typedef struct {
 enum { CB_FACTOR_FUSED = 0, CB_FACTOR_SPLIT = 1 };
 
 /* Schedules of the band solves' forward and backward sweeps (the same
- * solution up to rounding), all one tile row per workgroup: a chain step of
- * one 64x64 product with the matrix Linv_I L_{I,I-1} formed after each
- * factorization (default), of two dependent 64x64 products, or both sweeps on
- * a look-ahead system whose rows depend on the rows two and more back, its
- * band (twice the memory of the factor's) formed after each factorization:
- * faster sweeps for the drivers that solve many times per factorization
- * (arc length, modified NR).  CB_SWEEP_LOOK3 deepens that system once more
- * (rows three and more back, by substituting row I-2's equation into row I;
- * one more band each way). */
+ * solution up to rounding): blocks of four tile rows, with the block inverses
+ * and the links between neighbouring blocks formed after each factorization
+ * (CB_SWEEP_CHAIN, the default), or one tile row at a time with two dependent
+ * 64x64 products per row and nothing formed (CB_SWEEP_ROWS).  CB_SWEEP_LOOK2 and
+ * CB_SWEEP_LOOK3 named systems that decoupled neighbouring tile rows; the blocks
+ * are faster than both and serve them. */
 enum { CB_SWEEP_CHAIN = 0, CB_SWEEP_ROWS = 1, CB_SWEEP_LOOK2 = 2, CB_SWEEP_LOOK3 = 3 };
 
 /* Generations of the per-element state (base = last converged, _i = current
@@ -113,8 +110,8 @@ enum { CB_GEN_BASE = 0, CB_GEN_I = 1, CB_GEN_IP = 2 };
 
 /* Kernel families of the band solver (timed with HIP events on their stream):
  * the fused factorization launch (per tile column), the diag/panel/update launches
- * of the split schedule, the forward and backward sweeps, and the launch that
- * forms the sweeps' chain matrices after a factorization. */
+ * of the split schedule, the forward and backward sweeps, and the launches
+ * that form the sweeps' block matrices after a factorization. */
 enum { CB_KT_COLUMN = 0, CB_KT_DIAG = 1, CB_KT_PANEL = 2, CB_KT_UPDATE = 3, CB_KT_FWD = 4, CB_KT_BWD = 5,
        CB_KT_PREP = 6, CB_KT_N = 7 };
 
