@@ -60,9 +60,13 @@ struct BandLDLT {
     // Linv_B^T L_{B+1,B}^T [nt][4], formed after each factorization; the
     // right-hand side [nt * 64] and the helpers' partial sums; allocated at the
     // first factorization that needs them
-    bool chained = true;     // block sweeps (default) or the two-product row step
-    // a band of at most one block of four tile rows takes the row step
-    bool blocked() const { return chained && nt > 4; }
+    bool chained = true;     // sweeps with formed matrices, or the two-product row step
+    int look = 0;            // with chained: 2 or 3, the block sweeps
+    bool blocked() const { return chained && look >= 2 && nt > 4; }
+    // otherwise the chain matrices M_I = Linv_I L_{I,I-1} and G_I = L_{I+1,I}
+    // Linv_I, [nt] tiles each, allocated at the first factorization too
+    R* cmat = nullptr;
+    R* gmat = nullptr;
     R* lb = nullptr;
     R* mch = nullptr;
     R* gch = nullptr;

@@ -312,99 +312,47 @@ template <> struct SymAcc<double> : LowerAcc { static constexpr int N = 8; };
 // ---- D_K --------------------------------------------------------------------
 // The task takes the 64x64 tile S (lower part; the part above the diagonal is
 // never read) in LDS as xs[col][row], writes D to piv and Linv = L^{-1} (zeros
-// above the diagonal) to lout, and overwrites xs and ys.  L_KK itself is read
-// by neither the panels and updates nor the solves and is not stored.  FP32
+// above the diagonal) to lout, and overwrites xs.  L_KK itself is read by
+// neither the panels and updates nor the solves and is not stored.  FP32
 // tiles go through the FP64 task (below).
-//
-// FP64, blocked by 16: [S | I] is eliminated by block columns k = 0..3.
-//  - Wavefront 0 runs the 16 pivot steps of block column k in its registers.
-//    Each of its four 16-lane rows holds the 16x16 diagonal block (lane j:
-//    row j, a[c] = A_jc) and one 16x16 block of right-hand sides of the same
-//    elimination (lane j: x[c], c = 0..15).  Row g carries block (k + g) mod 4:
-//    the identity for g = 0, which becomes Linv_kk; A_ik^T for a block row i
-//    below, which becomes (L_ik D_k)^T; and for a block column j to the left
-//    B_kj = -sum_{m<k} L_km Linv_mj, which becomes Linv_kj.  So the four rows
-//    always have one block each and Linv is complete with the last pivot.
-//    Step c needs a[c] alone: the pivot and the factor of row i are its lanes
-//    c and i, which reach the whole 16-lane row as DPP operands (row_newbcast)
-//    of the FP64 multiply-adds.  The next pivot is formed first and its
-//    reciprocal while the rest of the step issues.
-//  - After a barrier wavefronts 0..3 update what block column k + 1 needs
-//    (FP64 MFMA 16x16x4, four steps per 16x16 block); the blocks of the later
-//    columns follow on the other wavefronts during the next pivot steps,
-//    except wavefront 4, which shares a SIMD with wavefront 0.
-// xs column 16k + c receives -L_ik in rows 16i.. (and -x/d elsewhere), ys row
-// 16k + c the right-hand sides: Linv row by row up to the diagonal and L D
-// beyond it.  Multipliers are l = a / d as a * (1/d), with the reciprocal's
-// correction applied to the product.
-// What bounds it is the chain of 64 pivots: reciprocal (28 cycles), its
-// correction, multiplier and next pivot (8 cycles an FP64 operation), and 5.5
-// cycles for each of a step's up to 30 multiply-adds.  One tile on an idle GPU
-// takes 7.3 us; with the columns broadcast through LDS, the blocks of Linv
-// formed beside and after the pivots, it took 12.1 us (pivots then came at 370
-// cycles each, now at about 190).
 template <class R> struct DiagScratch;
-template <> struct DiagScratch<double> { double dg[16][16]; };   // a[c] of every lane when column c's pivot is taken
+template <> struct DiagScratch<double> { double tsc[5][256]; double ub[16]; };
+// FP64: blocked by 16.  For each column block k:
+//  - wavefront 0 factorizes the 64x16 panel (rows 16k..63, lane = row):
+//    16 pivot steps, each broadcasting column c of the block through LDS; the
+//    pivot and the next step's critical entry travel by readlane, and the
+//    reciprocal of the next pivot is formed while the rest of the step's
+//    updates are issued.  The block lanes also form column p of Linv_kk by
+//    the same elimination applied to the identity.  Multipliers are
+//    l = a * (1/d) with the reciprocal refined by two Newton steps.
+//  - the other wavefronts meanwhile form the off-diagonal blocks of Linv
+//    that are ready, Linv_ij = -Linv_ii sum_{k=j}^{i-1} L_ik Linv_kj, as
+//    16x16x16 FP64 MFMA products, avoiding wavefront 4 (which shares a SIMD
+//    with wavefront 0);
+//  - after a barrier, up to six wavefronts update the trailing blocks
+//    A_ij -= L_ik D_k L_jk^T (16x16x16 FP64 MFMA).
+// Linv is kept in ys column-major with the row index swizzled by the column
+// (ysw), which makes both row and column accesses free of bank conflicts.
 
-// ys index of row c, column r: the columns of a row are permuted so that both
-// rows and columns are read without bank conflicts
-__device__ __forceinline__ int ysw(int c, int r) { return c * T + (r ^ ((c & 3) << 4 | (c >> 2 & 15))); }
+__device__ __forceinline__ int ysw(int col, int row) { return col * T + (row ^ (col & 15)); }
 
-// The pivot steps' operations are volatile so that they issue in the order
-// written: a DPP operand must not have been written by either of the two
-// instructions in front.
-template <int I> __device__ __forceinline__ void fmac_lane(double& acc, double ac, double m) {   // acc += ac(lane I) m
-    __asm__ volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
-                     : "+v"(acc) : "v"(ac), "v"(m), "n"(I));
-}
-template <int I, int E>
-__device__ __forceinline__ void fmac_lanes(double* a, double* x, double ac, double m, double l) {   // i = I .. E-1
-    if constexpr (I < E && I < 16) {
-        fmac_lane<I>(a[I], ac, m);
-        fmac_lane<I>(x[I], ac, l);
-        fmac_lanes<I + 1, E>(a, x, ac, m, l);
-    }
-}
-template <int C> __device__ __forceinline__ double row_lane(double v) {   // v of lane C
-    double r;
-    __asm__ volatile("v_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(v), "n"(C));
-    return r;
+__device__ __forceinline__ double recip(double d) {
+    double r = __builtin_amdgcn_rcp(d);
+    double e = __builtin_fma(-d, r, 1.0);
+    r = __builtin_fma(r, e, r);
+    e = __builtin_fma(-d, r, 1.0);
+    return __builtin_fma(r, e, r);
 }
 
-// Steps C .. 15: r is 1/d of pivot d = a[C] (lane C) to a relative error e
-// below 2^-23 and e2 = e + e^2, so that 1/d is r + r e2; q = a[C] r.  xs, dg:
-// this lane's
-// entry of row 0 of the block and of the pivot columns; off: its byte offset
-// in a row of ys before the row's permutation.
-template <int C>
-__device__ __forceinline__ void pivot_steps(double* a, double* x, double r, double q, double e2, double* xs, char* ysb,
-                                            int off, double* dg) {
-    const double ac = a[C], xc = x[C];
-    double m, l, rd;
-    __asm__ volatile("v_fma_f64 %0, -%1, %2, -%1" : "=v"(m) : "v"(q), "v"(e2));          // -a[C] / d
-    __asm__ volatile("v_fma_f64 %0, -%1, %2, -%1" : "=v"(rd) : "v"(r), "v"(e2));         // -1 / d
-    if constexpr (C < 15) fmac_lane<C + 1>(a[C + 1], ac, m);
-    __asm__ volatile("v_mul_f64 %0, %1, %2" : "=v"(l) : "v"(xc), "v"(rd));               // -x[C] / d
-    double rn = 0.0, en = 0.0, qn = 0.0, e2n = 0.0;
-    if constexpr (C < 15) {
-        if constexpr (C < 14) fmac_lane<C + 2>(a[C + 2], ac, m);
-        else __asm__ volatile("s_nop 0");
-        const double dn = row_lane<C + 1>(a[C + 1]);
-        fmac_lane<C + 1>(x[C + 1], ac, l);
-        __asm__ volatile("v_rcp_f64 %0, %1" : "=v"(rn) : "v"(dn));
-        if constexpr (C < 14) fmac_lane<C + 2>(x[C + 2], ac, l);
-        fmac_lanes<C + 3, C + 5>(a, x, ac, m, l);
-        if constexpr (C > 12) __asm__ volatile("s_nop 0");
-        __asm__ volatile("v_fma_f64 %0, -%1, %2, 1.0" : "=v"(en) : "v"(dn), "v"(rn));
-        __asm__ volatile("v_mul_f64 %0, %1, %2" : "=v"(qn) : "v"(a[C + 1]), "v"(rn));
-        fmac_lanes<C + 5, C + 6>(a, x, ac, m, l);
-        __asm__ volatile("v_fma_f64 %0, %1, %1, %1" : "=v"(e2n) : "v"(en));
-        fmac_lanes<C + 6, 16>(a, x, ac, m, l);
-    }
-    xs[C * T] = l;
-    *reinterpret_cast<double*>(ysb + C * T * 8 + (off ^ ((C & 3) << 7 | C >> 2 << 3))) = xc;
-    dg[C * 16] = ac;
-    if constexpr (C < 15) pivot_steps<C + 1>(a, x, rn, qn, e2n, xs, ysb, off, dg);
+// D[m][n] = sum_t A(m, t) B(t, n) over 16x16 blocks on one wavefront (FP64
+// MFMA 16x16x4: lane l supplies A(l%16, t) and B(t, l%16), t = t0 + l/16);
+// element e of lane l is D[l/16 + 4e][l%16].
+template <class FA, class FB>
+__device__ __forceinline__ d4 mm16(FA A, FB B, d4 acc) {
+    const int l = threadIdx.x & 63, rr = l & 15, lg = l >> 4;
+#pragma unroll
+    for (int t0 = 0; t0 < 16; t0 += 4) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A(rr, t0 + lg), B(t0 + lg, rr), acc, 0, 0, 0);
+    return acc;
 }
 
 struct NoSide {
@@ -412,84 +360,162 @@ struct NoSide {
 };
 
 // side(k, wv) runs on every wavefront in each block column's phase, on
-// wavefront 0 before the pivot steps and on the others beside them (after the
-// trailing blocks they may have).  LDS_ONLY: Linv goes to lds_out alone and D
-// stays in dd; the caller stores them.
+// wavefront 0 before the pivot steps and on the others beside them (after
+// their own products), and on all of them once more, with k = 4, before the
+// last products.  LDS_ONLY: Linv goes to lds_out alone and D stays in
+// dd; the caller stores them.
 template <bool LDS_ONLY = false, class O = double, class Side = NoSide>
 __device__ __forceinline__ void diag_task(double (*xs)[T], double* ys, double* dd, DiagScratch<double>& sm,
                                           O* __restrict__ lout, double* __restrict__ piv, long Kt,
                                           O* lds_out = nullptr, Side side = Side()) {
-    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, rr = l & 15, lg = l >> 4;
-    // block (q, p) of the elimination after block column m: A_qp (q >= p > m)
-    // or B_pq (q <= m; its first contribution when q = m)
-    // (the sixteen products are summed before they meet the entry, which
-    // costs one rounding at its magnitude instead of four)
-    auto trail = [&](int m, int p, int q) {
-        d4 old = {0.0, 0.0, 0.0, 0.0}, acc = old;
-        if (q != m) {
+    const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, rr = l & 15, lg = l >> 4;
+    double(*tsc)[256] = sm.tsc;
+    // operand views: L_ik (rows r, cols t), Linv_ij as (t, c) and as (r, t), T slot s as (t, c)
+    auto Lb = [&](int i, int k) { return [&, i, k](int r, int t) { return xs[16 * k + t][16 * i + r]; }; };
+    auto Vb = [&](int i, int j) { return [&, i, j](int t, int c) { return ys[ysw(16 * j + c, 16 * i + t)]; }; };
+    auto Vr = [&](int i, int j) { return [&, i, j](int r, int t) { return ys[ysw(16 * j + t, 16 * i + r)]; }; };
+    auto Tb = [&](int s) { return [&, s](int t, int c) { return tsc[s][t * 16 + c]; }; };
+    auto getT = [&](int s) {
+        d4 acc;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) old[e] = xs[16 * p + lg + 4 * e][16 * q + rr];
-        }
-#pragma unroll
-        for (int t0 = 0; t0 < 16; t0 += 4) {
-            const int t = 16 * m + t0 + lg;
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(xs[t][16 * p + rr], ys[ysw(t, 16 * q + rr)], acc, 0, 0, 0);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) xs[16 * p + lg + 4 * e][16 * q + rr] = old[e] + acc[e];
+        for (int e = 0; e < 4; ++e) acc[e] = tsc[s][(lg + 4 * e) * 16 + rr];
+        return acc;
     };
+    auto putT = [&](int s, d4 acc) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tsc[s][(lg + 4 * e) * 16 + rr] = acc[e];
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto putV = [&](int i, int j, d4 acc) {   // Linv_ij = -acc
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ys[ysw(16 * j + rr, 16 * i + lg + 4 * e)] = -acc[e];
+        __builtin_amdgcn_wave_barrier();
+    };
+    const d4 z = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll 1
     for (int k = 0; k < 4; ++k) {
         if (wv == 0) {
             side(k, 0);
-            const int base = 16 * k, row = 16 * ((k + lg) & 3) + rr;
-            double a[16], x[16];
+            const int r = l, base = 16 * k, p = r - base;
+            double v[16], bcol[16];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                v[q] = xs[base + q][r];
+                bcol[q] = (q == p) ? 1.0 : 0.0;
+            }
+            if (p >= 0 && p < 16) sm.ub[p] = v[0];
+            __builtin_amdgcn_wave_barrier();
+            double d = lane_value(v[0], base);
+            double rd = recip(d);
+            double dr = 0.0;
+            double U[16];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) U[q] = sm.ub[q];
 #pragma unroll
             for (int c = 0; c < 16; ++c) {
-                a[c] = xs[base + c][base + rr];
-                x[c] = xs[base + c][row];
-            }
+                int po = p;
+                __asm__ volatile("" : "+v"(po));   // keeps the per-step lane tests in the step
+                const bool below = po > c;
+                dr = (po == c) ? d : dr;
+                const double le = below ? v[c] * rd : 0.0;
+                const double fb = below ? 0.0 : bcol[c] * rd;
+                double dn = 0.0, rdn = 0.0, un = 0.0;
+                if (c + 1 < 16) {
+                    v[c + 1] = __builtin_fma(-le, U[c + 1], v[c + 1]);
+                    __builtin_amdgcn_wave_barrier();
+                    if (po >= 0 && po < 16) sm.ub[po] = v[c + 1];
+                    __builtin_amdgcn_wave_barrier();
+                    dn = lane_value(v[c + 1], base + c + 1);
+                    if (c + 2 < 16) un = lane_value(v[c + 1], base + c + 2);
+                    rdn = recip(dn);
+                }
 #pragma unroll
-            for (int c = 0; c < 16; ++c) x[c] = (lg == 0) ? (c == rr ? 1.0 : 0.0) : x[c];
-            __asm__ volatile("s_nop 1" : "+v"(a[0]));
-            const double d = row_lane<0>(a[0]), r = __builtin_amdgcn_rcp(d), e = __builtin_fma(-d, r, 1.0);
-            pivot_steps<0>(a, x, r, a[0] * r, __builtin_fma(e, e, e), &xs[base][row],
-                           reinterpret_cast<char*>(ys + base * T), (row ^ 4 * k) * 8, &sm.dg[0][rr]);
-            if (l < 16) dd[base + l] = sm.dg[l][l];
-        } else {
-            if (k == 1) {   // after block column 0: blocks of the columns 2 and 3
-                if (wv == 1) trail(0, 2, 0);
-                else if (wv == 2) trail(0, 2, 2);
-                else if (wv == 3) trail(0, 2, 3);
-                else if (wv == 5) trail(0, 3, 0);
-                else if (wv == 6) trail(0, 3, 3);
-            } else if (k == 2) {
-                if (wv == 1) trail(1, 3, 0);
-                else if (wv == 2) trail(1, 3, 1);
-                else if (wv == 3) trail(1, 3, 3);
+                for (int q = c + 2; q < 16; ++q) v[q] = __builtin_fma(-le, U[q], v[q]);
+#pragma unroll
+                for (int q = c + 1; q < 16; ++q) bcol[q] = __builtin_fma(-fb, U[q], bcol[q]);
+                v[c] = below ? le : v[c];
+                if (c + 1 < 16) {
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) U[q] = (q == c + 2) ? un : sm.ub[q];
+                    d = dn;
+                    rd = rdn;
+                }
+                // keep every update in its own step (no deferred chains)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    __asm__ volatile("" : "+v"(v[q]));
+                    __asm__ volatile("" : "+v"(bcol[q]));
+                }
             }
-            side(k, wv);
+            if (p >= 0) {
+#pragma unroll
+                for (int q = 0; q < 16; ++q) xs[base + q][r] = v[q];
+            }
+            if (p >= 0 && p < 16) {
+                dd[r] = dr;
+                if (!LDS_ONLY) piv[Kt * T + r] = dr;
+#pragma unroll
+                for (int q = 0; q < 16; ++q) ys[ysw(base + p, base + q)] = (q >= p) ? bcol[q] : 0.0;
+            }
+        } else if (k == 1) {
+            if (wv == 1) putT(0, mm16(Lb(1, 0), Vb(0, 0), z));                      // T_10
+        } else if (k == 2) {
+            if (wv == 1) {
+                putV(1, 0, mm16(Vr(1, 1), Tb(0), z));                                // Linv_10
+                putT(1, mm16(Lb(2, 1), Vb(1, 0), mm16(Lb(2, 0), Vb(0, 0), z)));      // T_20
+            } else if (wv == 2) {
+                putT(2, mm16(Lb(2, 1), Vb(1, 1), z));                                // T_21
+            } else if (wv == 3) {
+                putT(3, mm16(Lb(3, 0), Vb(0, 0), z));                                // T_30, first term
+            } else if (wv == 5) {
+                putT(4, mm16(Lb(3, 1), Vb(1, 1), z));                                // T_31, first term
+            }
+        } else if (k == 3) {
+            if (wv == 1) putV(2, 0, mm16(Vr(2, 2), Tb(1), z));                       // Linv_20
+            else if (wv == 2) putV(2, 1, mm16(Vr(2, 2), Tb(2), z));                  // Linv_21
+            else if (wv == 3) putT(3, mm16(Lb(3, 1), Vb(1, 0), getT(3)));            // T_30, second term
+            else if (wv == 5) putT(0, mm16(Lb(3, 2), Vb(2, 2), z));                  // T_32
+        }
+        if (wv != 0) side(k, wv);
+        __syncthreads();
+        if (k == 3) break;
+        // trailing update of the blocks k < j <= i <= 3, one per wavefront
+        {
+            const int nb = 3 - k;
+            int pp = wv, i = -1, j = -1;
+            for (int a = 0; a < nb && i < 0; ++a)
+                for (int b = 0; b <= a; ++b) {
+                    if (pp == 0) { i = k + 1 + a; j = k + 1 + b; break; }
+                    --pp;
+                }
+            if (i >= 0) {
+                // D[m = c][n = r] = sum_t L_jk[c][t] (L_ik[r][t] d_t)
+                const d4 acc = mm16([&](int c, int t) { return xs[16 * k + t][16 * j + c]; },
+                                    [&](int t, int r) { return xs[16 * k + t][16 * i + r] * dd[16 * k + t]; }, z);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) xs[16 * j + lg + 4 * e][16 * i + rr] -= acc[e];
+            }
         }
         __syncthreads();
-        if (k < 3) {
-            if (wv < 4) trail(k, k + 1, wv);
-            __syncthreads();
-        }
     }
-    // Linv, column-major: all reads before the first store (one at a time took
-    // 1.5 us)
-    O v[TT / NTH];
-#pragma unroll
-    for (int i = 0; i < TT / NTH; ++i) {
-        const int idx = tid + NTH * i, col = idx / T, row = idx % T;
-        v[i] = O((row >= col) ? ys[ysw(row, col)] : 0.0);
+    side(4, wv);
+    // the last row of blocks: T_3j completed, Linv_3j = -Linv_33 T_3j
+    if (wv == 0) {
+        putT(1, mm16(Lb(3, 2), Vb(2, 0), getT(3)));
+        putV(3, 0, mm16(Vr(3, 3), Tb(1), z));
+    } else if (wv == 1) {
+        putT(2, mm16(Lb(3, 2), Vb(2, 1), getT(4)));
+        putV(3, 1, mm16(Vr(3, 3), Tb(2), z));
+    } else if (wv == 2) {
+        putV(3, 2, mm16(Vr(3, 3), Tb(0), z));
     }
-#pragma unroll
-    for (int i = 0; i < TT / NTH; ++i) {
-        if (!LDS_ONLY) lout[tid + NTH * i] = v[i];
-        if (LDS_ONLY || lds_out) lds_out[tid + NTH * i] = v[i];
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < TT; idx += NTH) {
+        const int col = idx / T, row = idx % T;
+        const double v = (row >= col) ? ys[ysw(col, row)] : 0.0;
+        if (!LDS_ONLY) lout[idx] = O(v);
+        if (LDS_ONLY || lds_out) lds_out[idx] = O(v);
     }
-    if (!LDS_ONLY && wv == 0) piv[Kt * T + l] = dd[l];
 }
 
 // FP32 tiles: the FP64 task on the tile widened in LDS, with Linv rounded once
@@ -638,11 +664,10 @@ __global__ void __launch_bounds__(NTH) k_tile_update(R* __restrict__ tiles, cons
 //   corner(I)  (I, I) likewise, with P_{I,I-2}
 // One column's critical path is then the chain's own P, U, D or half the loop
 // Linv_{J-2} -> near(J) -> chain -> Linv_J, whichever is longer.  The chain is:
-// 12.6 us a column whatever the band's width up to 25 tiles (panel 2.6, first
-// diagonal blocks 0.9, diagonal task 8.2, hand-over 0.9), against 21.2 us for
-// a launch per column whose workgroups loaded and stored every tile they
-// updated.  The workgroups of a band of 25 tiles need about 3 us a column of
-// the whole chip's matrix units, so they keep up.  Counters (zero
+// 17.9 us a column (200 x 200 panel, 12.1 of it the diagonal task), against
+// 21.2 us for a launch per column whose workgroups loaded and stored every
+// tile they updated.  The other workgroups of a band of 25 tiles need about 3 us
+// a column of the whole chip's matrix units, so they keep up.  Counters (zero
 // before the launch): P_ROW the columns of a tile row that its tile() tasks have
 // finished, P_LAST L_{J,J-1} stored, P_DIAG D_J and Linv_J stored, P_NEAR and
 // P_NEAR2 a row's two last tiles handed over, P_PART tile (I, I-2) handed over (in
@@ -1233,10 +1258,202 @@ __global__ void __launch_bounds__(256) k_bwd_sweep(const R* __restrict__ tiles_t
     if (tid < T) put_value(&x[I * T + tid], part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid]);
 }
 
+// ---- sweeps with a precomputed chain matrix ----------------------------------
+// In the sweeps above the last step of a tile row waits for its predecessor
+// and then applies two dependent 64x64 products (L_{I,I-1} y_{I-1}, then Linv_I).
+// After each factorization k_sweep_chain forms per tile row
+//   M_I = Linv_I L_{I,I-1}            (column-major, for the forward sweep)
+//   G_I = L_{I+1,I} Linv_I            (row-major, for the backward sweep)
+// so that y_I = U_I - M_I y_{I-1}, U_I = Linv_I (b_I - sum_{J <= I-2} L_IJ y_J),
+// and x_I = U'_I - G_I^T x_{I+1}, U'_I = Linv_I^T (y_I / D_I - sum_{J >= I+2} L_JI^T x_J).
+// U_I needs the rows up to I-2 only, which arrive one chain step before
+// y_{I-1}; once y_{I-1} lands the row takes one 64x64 product and one
+// reduction.  Each workgroup still reads only its own tile row (the older
+// contributions' bandwidth per workgroup is that of the sweeps above).
+
+// tile (I, J) of the factor, I > J, read as doubles; zero outside the band
+template <class R> struct TileRd {
+    const R* p;
+    __device__ double operator()(int r, int c) const { return p ? double(p[c * T + r]) : 0.0; }
+};
+template <class R> __device__ inline TileRd<R> factor_tile(const R* tiles, long I, long J, long nt, int w) {
+    if (J < 0 || I >= nt || I - J > w || I - J < 1) return TileRd<R>{nullptr};
+    return TileRd<R>{tiles + tile_index(I, J, w) * TT};
+}
+template <class R> __device__ inline TileRd<R> linv_tile(const R* linv, long I, long nt) {
+    return TileRd<R>{(I >= 0 && I < nt) ? linv + I * TT : nullptr};
+}
+
+// acc[j] += sum_k A(r, k) B(k, c0 + j), j < 16 (B's reads are uniform over a wavefront)
+template <class FA, class FB> __device__ inline void mm64(const FA& A, const FB& B, int r, int c0, double* acc) {
+    for (int k = 0; k < T; ++k) {
+        const double a = A(r, k);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[j] += a * B(k, c0 + j);
+    }
+}
+
+// M_I and G_I for every tile row: one workgroup per row, thread (r, c0)
+// forming entries (r, c0..c0+15) of each product.
+template <class R>
+__global__ void __launch_bounds__(256) k_sweep_chain(const R* __restrict__ tiles, const R* __restrict__ linv,
+                                                     R* __restrict__ mch, R* __restrict__ gch, long nt, int w) {
+    const long I = blockIdx.x;
+    const int r = threadIdx.x % T, c0 = 16 * (threadIdx.x / T);
+    double acc[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[j] = 0.0;
+    mm64(linv_tile(linv, I, nt), factor_tile(tiles, I, I - 1, nt, w), r, c0, acc);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) mch[I * TT + (c0 + j) * T + r] = R(acc[j]);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[j] = 0.0;
+    mm64(factor_tile(tiles, I + 1, I, nt, w), linv_tile(linv, I, nt), r, c0, acc);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) gch[I * TT + r * T + c0 + j] = R(acc[j]);
+}
+
+// y_I = U_I - M_I y_{I-1}.  r is read from xr, whose slot I is set to SENT for
+// the backward sweep; y must hold SENT.
+template <class R>
+__global__ void __launch_bounds__(256) k_fwd_sweep_m(const R* __restrict__ tiles, const R* __restrict__ linv,
+                                                     const R* __restrict__ mch, double* __restrict__ xr, double* y,
+                                                     long nt, int w, long spin_limit, int* err) {
+    __shared__ double vin[T];
+    __shared__ double vch[NCH][T];
+    __shared__ double part[4][T];
+    const long I = blockIdx.x;
+    const int tid = threadIdx.x, row = tid % T, q = tid / T, k0 = 16 * q;
+    R lv[16], lm[16];
+    const R* lvp = linv + I * (long)TT;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) lv[k] = lvp[(k0 + k) * T + row];
+    const bool has_prev = I >= 1;
+    if (has_prev) {
+        const R* lmp = mch + I * (long)TT;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) lm[k] = lmp[(k0 + k) * T + row];
+    }
+    double acc = 0.0;
+    if (q == 0) {
+        acc = xr[I * T + row];
+        xr[I * T + row] = __builtin_bit_cast(double, SENT);
+    }
+    // the older rows J <= I - 2 in chunks of NCH, wavefront c polling row J + c
+    const long J0 = I - w > 0 ? I - w : 0;
+    for (long J = J0; J < I - 1; J += NCH) {
+        const int nc = (I - 1 - J < NCH) ? int(I - 1 - J) : NCH;
+        R lx[NCH][16];
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+            if (c < nc) {
+                const R* l = tiles + (I * (w + 1) + (J + c - I + w)) * (long)TT;
+#pragma unroll
+                for (int k = 0; k < 16; ++k) lx[c][k] = l[(k0 + k) * T + row];
+            }
+        fetch_rows(y, J, 1, nc, vch, spin_limit, err);
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+            if (c < nc) {
+#pragma unroll
+                for (int k = 0; k < 16; ++k) acc -= double(lx[c][k]) * vch[c][k0 + k];
+            }
+        __syncthreads();
+    }
+    // U_I = Linv_I S_I, formed before y_{I-1} is needed
+    part[q][row] = acc;
+    __syncthreads();
+    if (tid < T) vin[tid] = part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid];
+    __syncthreads();
+    double u = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) u += double(lv[k]) * vin[k0 + k];
+    __syncthreads();
+    part[q][row] = u;
+    __syncthreads();
+    double yi = (q == 0) ? part[0][row] + part[1][row] + part[2][row] + part[3][row] : 0.0;
+    if (has_prev) {
+        fetch_row(y, I - 1, vin, spin_limit, err);
+        double m = 0.0;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) m += double(lm[k]) * vin[k0 + k];
+        part[q][row] = m;
+        __syncthreads();
+        if (q == 0) yi -= part[0][row] + part[1][row] + part[2][row] + part[3][row];
+    }
+    if (q == 0) put_value(&y[I * T + row], yi);
+}
+
+// x_I = U'_I - G_I^T x_{I+1}; workgroup g handles I = nt-1-g.  x must hold SENT.
+template <class R>
+__global__ void __launch_bounds__(256) k_bwd_sweep_m(const R* __restrict__ tiles_t, const R* __restrict__ linv,
+                                                     const R* __restrict__ gch, const double* __restrict__ y,
+                                                     const double* __restrict__ piv, double* x, long nt, int w,
+                                                     long spin_limit, int* err) {
+    __shared__ double vin[T];
+    __shared__ double vch[NCH][T];
+    __shared__ double part[4][T];
+    const long I = nt - 1 - blockIdx.x;
+    const int tid = threadIdx.x, col = tid % T, q = tid / T, k0 = 16 * q;
+    R lv[16], lm[16];
+    const R* lvp = linv + I * (long)TT;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) lv[k] = lvp[col * T + k0 + k];   // Linv[k][col]
+    const bool has_next = I + 1 < nt;
+    if (has_next) {
+        const R* lgp = gch + I * (long)TT;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) lm[k] = lgp[(k0 + k) * T + col];   // G_I[k][col]
+    }
+    double acc = (q == 0) ? y[I * T + col] / piv[I * T + col] : 0.0;
+    // the later rows J >= I + 2 in chunks of NCH, wavefront c polling row J - c
+    const long J1 = (I + w < nt - 1) ? I + w : nt - 1;
+    for (long J = J1; J > I + 1; J -= NCH) {
+        const int nc = (J - (I + 1) < NCH) ? int(J - (I + 1)) : NCH;
+        R lx[NCH][16];
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+            if (c < nc) {
+                const R* l = tiles_t + ((J - c) * (w + 1) + (I - (J - c) + w)) * (long)TT;
+#pragma unroll
+                for (int k = 0; k < 16; ++k) lx[c][k] = l[(k0 + k) * T + col];
+            }
+        fetch_rows(x, J, -1, nc, vch, spin_limit, err);
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+            if (c < nc) {
+#pragma unroll
+                for (int k = 0; k < 16; ++k) acc -= double(lx[c][k]) * vch[c][k0 + k];
+            }
+        __syncthreads();
+    }
+    part[q][col] = acc;
+    __syncthreads();
+    if (tid < T) vin[tid] = part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid];
+    __syncthreads();
+    double u = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) u += double(lv[k]) * vin[k0 + k];
+    __syncthreads();
+    part[q][col] = u;
+    __syncthreads();
+    double xi = (q == 0) ? part[0][col] + part[1][col] + part[2][col] + part[3][col] : 0.0;
+    if (has_next) {
+        fetch_row(x, I + 1, vin, spin_limit, err);
+        double m = 0.0;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) m += double(lm[k]) * vin[k0 + k];
+        part[q][col] = m;
+        __syncthreads();
+        if (q == 0) xi -= part[0][col] + part[1][col] + part[2][col] + part[3][col];
+    }
+    if (q == 0) put_value(&x[I * T + col], xi);
+}
+
 // ---- block sweeps --------------------------------------------------------------
 // Above, every tile row waits for the one before: about 1 us a row of store,
-// poll and products, however fast the tiles stream.  The default schedule
-// takes SB tile rows at a time.  With Linv_B the inverse of a block's SB x SB
+// poll and products, however fast the tiles stream.  The look-ahead schedules
+// take SB tile rows at a time.  With Linv_B the inverse of a block's SB x SB
 // tiles of L, formed after each factorization,
 //   y_B = Linv_B S_B - M_B y_{B-1},  S_B = b_B - sum over the rows before block B-1,
 //   M_B = Linv_B L_{B,B-1},
@@ -1255,7 +1472,7 @@ __global__ void __launch_bounds__(256) k_bwd_sweep(const R* __restrict__ tiles_t
 // factorization; one row at a time took 6.2 / 6.5 ms, and systems that
 // decoupled each row from the one or two before 5.1 / 5.2 ms with 11 ms of
 // forming.  A band of a single block has nothing to overlap and takes the
-// row sweeps, which need nothing formed (BandLDLT::blocked).
+// chain matrices (BandLDLT::blocked).
 constexpr int SB = 4;      // tile rows per block
 constexpr int HT = 8;      // tiles per helper; a wavefront polls one of their rows
 constexpr int SWT = 512;
@@ -1596,7 +1813,7 @@ __global__ void __launch_bounds__(NTH) k_band_factor_models(double* __restrict__
         }
         staged = false;
         diag_task(xs, ys, dd, sm, linv + K * (long)TT, piv, K, &lk[0][0], [&](int k, int) {
-            if (pre && k == 3) {
+            if (pre && k == 4) {
                 const double* t1 = tiles + tile_index(K + 1, K, w) * TT;
 #pragma unroll
                 for (int i = 0; i < TT / NTH; ++i) pa[i] = t1[threadIdx.x + NTH * i];
@@ -1919,10 +2136,11 @@ void BandLDLT<R>::setup(long n_, long bandwidth, hipStream_t s_) {
 
 template <class R>
 void BandLDLT<R>::release() {
-    void* ps[] = {tiles, tiles_t, linv, lb, mch, gch, piv, xw, yw, bw, part, flag, prog};
+    void* ps[] = {tiles, tiles_t, linv, lb, mch, gch, cmat, gmat, piv, xw, yw, bw, part, flag, prog};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     tiles = nullptr; tiles_t = nullptr; linv = nullptr; piv = nullptr; xw = nullptr; yw = nullptr; flag = nullptr;
+    cmat = nullptr; gmat = nullptr;
     lb = nullptr; mch = nullptr; gch = nullptr; bw = nullptr; part = nullptr;
     prog = nullptr;
     clock.release();
@@ -1976,6 +2194,17 @@ int BandLDLT<R>::factor(const Dev& d) {
         }
     }
     CB_CHECK(hipGetLastError());
+    if (chained && !blocked()) {
+        if (!cmat) {
+            cmat = dalloc<R>(size_t(nt) * TT);
+            gmat = dalloc<R>(size_t(nt) * TT);
+        }
+        const bool tk_prep = clock.take(KT_PREP);
+        if (tk_prep) clock.begin(KT_PREP, s);
+        hipLaunchKernelGGL((k_sweep_chain<R>), dim3(int(nt)), dim3(256), 0, s, tiles, linv, cmat, gmat, nt, w);
+        if (tk_prep) clock.end(s);
+        CB_CHECK(hipGetLastError());
+    }
     if (blocked()) {
         const bool tk_prep = clock.take(KT_PREP);
         if (tk_prep) clock.begin(KT_PREP, s);
@@ -2023,6 +2252,9 @@ void BandLDLT<R>::solve(const double* rhs, double* out) {
     if (blocked())
         hipLaunchKernelGGL((k_sweep_block<R, true>), dim3(grid), dim3(SWT), 0, s, tiles, linv, lb, mch, bw, piv, yw,
                            part, nt, w, gh, spin_limit, flag);
+    else if (chained)
+        hipLaunchKernelGGL((k_fwd_sweep_m<R>), dim3(int(nt)), dim3(256), 0, s, tiles, linv, cmat, xw, yw, nt, w,
+                           spin_limit, flag);
     else
         hipLaunchKernelGGL((k_fwd_sweep<R>), dim3(int(nt)), dim3(256), 0, s, tiles, linv, xw, yw, nt, w, spin_limit,
                            flag);
@@ -2032,6 +2264,9 @@ void BandLDLT<R>::solve(const double* rhs, double* out) {
     if (blocked())
         hipLaunchKernelGGL((k_sweep_block<R, false>), dim3(grid), dim3(SWT), 0, s, tiles_t, linv, lb, gch, yw, piv, xw,
                            part + npart, nt, w, gh, spin_limit, flag);
+    else if (chained)
+        hipLaunchKernelGGL((k_bwd_sweep_m<R>), dim3(int(nt)), dim3(256), 0, s, tiles_t, linv, gmat, yw, piv, xw, nt, w,
+                           spin_limit, flag);
     else
         hipLaunchKernelGGL((k_bwd_sweep<R>), dim3(int(nt)), dim3(256), 0, s, tiles_t, linv, yw, piv, xw, nt, w,
                            spin_limit, flag);

@@ -95,12 +95,13 @@ typedef struct {
 enum { CB_FACTOR_FUSED = 0, CB_FACTOR_SPLIT = 1 };
 
 /* Schedules of the band solves' forward and backward sweeps (the same
- * solution up to rounding): blocks of four tile rows, with the block inverses
- * and the links between neighbouring blocks formed after each factorization
- * (CB_SWEEP_CHAIN, the default), or one tile row at a time with two dependent
- * 64x64 products per row and nothing formed (CB_SWEEP_ROWS).  CB_SWEEP_LOOK2 and
- * CB_SWEEP_LOOK3 named systems that decoupled neighbouring tile rows; the blocks
- * are faster than both and serve them. */
+ * solution up to rounding): one tile row per workgroup with a chain step of
+ * one 64x64 product, the matrix Linv_I L_{I,I-1} formed after each factorization
+ * (CB_SWEEP_CHAIN, the default), or of two dependent 64x64 products
+ * (CB_SWEEP_ROWS), or blocks of four tile rows, with the block inverses and the
+ * links between neighbouring blocks formed after each factorization
+ * (CB_SWEEP_LOOK2 and CB_SWEEP_LOOK3, which named look-ahead systems before):
+ * less than half the time per solve. */
 enum { CB_SWEEP_CHAIN = 0, CB_SWEEP_ROWS = 1, CB_SWEEP_LOOK2 = 2, CB_SWEEP_LOOK3 = 3 };
 
 /* Generations of the per-element state (base = last converged, _i = current
