@@ -60,6 +60,9 @@ struct Dev {
     int32_t *blk_fr = nullptr, *col_el_fr = nullptr;
     int32_t *blkrow = nullptr, *gat_ptr_fr = nullptr, *gat_item_fr = nullptr;   // frame tangent gather
     int32_t *jnt_ptr_fr = nullptr, *jnt_item_fr = nullptr;                       // frame force gather
+    int32_t *jnt_ptr_tr = nullptr, *jnt_item_tr = nullptr;                       // bar force gather
+    int32_t *jnt_ptr_sh = nullptr, *jnt_item_sh = nullptr;                       // shell force gather
+    double* sh = nullptr;   // shell corner forces in global axes, 18 per shell
     double* fh = nullptr;   // frame end forces in global axes, 12 per member
     std::vector<int32_t> col_ptr_tr, col_ptr_sh, col_ptr_fr;
     // properties; llen, farea and slength are the working copies the element

@@ -271,20 +271,23 @@ __global__ void __launch_bounds__(128) k_shell_tangent(
         }
 }
 
-// Internal force of the shells of one colour (forces_sh ANAFLAG 2,
-// shell.c:1675-1786, 2305-2400).
+// Internal force of the shells (forces_sh ANAFLAG 2, shell.c:1675-1786,
+// 2305-2400): every shell in one launch leaves its global corner forces in h,
+// k_shell_forces_gather sums them.  A launch per colour that added into f
+// took the latency of one shell per colour (12 us each on a panel of 128
+// shells, 24 us on one of 131072 whose colours did not fill the chip).
 __global__ void __launch_bounds__(128) k_shell_forces(
-    const int32_t* __restrict__ els, int n, const int32_t* __restrict__ minc,
+    int n, const int32_t* __restrict__ minc,
     const int32_t* __restrict__ mcode, const double* __restrict__ x, const double* __restrict__ dd,
     const double* __restrict__ c1p, const double* __restrict__ c2p, const double* __restrict__ c3p,
     const double* __restrict__ c1c, const double* __restrict__ c2c, const double* __restrict__ c3c,
     const double* __restrict__ emod, const double* __restrict__ nu, const double* __restrict__ thick,
     const double* __restrict__ xlocal, const double* __restrict__ farea,
     const double* __restrict__ slength, double* __restrict__ ef_ip, double* __restrict__ ef_i,
-    double* __restrict__ f, long ioff, long toff, long poff, long moff, long eoff) {
+    double* __restrict__ h, long ioff, long toff, long poff, long moff, long eoff) {
     int it = blockIdx.x * blockDim.x + threadIdx.x;
     if (it >= n) return;
-    const long e = els[it];
+    const long e = it;
     const double E = emod[poff + e], v = nu[e], t = thick[e], A0 = farea[e];
     const double xl[3] = {xlocal[e * 3], xlocal[e * 3 + 1], xlocal[e * 3 + 2]};
     const double sl[3] = {slength[e * 3], slength[e * 3 + 1], slength[e * 3 + 2]};
@@ -367,16 +370,28 @@ __global__ void __launch_bounds__(128) k_shell_forces(
     for (int i = 0; i < 18; ++i) efo[i] = efc[i];
 #pragma unroll
     for (int a = 0; a < 3; ++a) { efp[6 * a] = 0.0; efp[6 * a + 1] = 0.0; }
-    // global force T_i^T ef_i scattered by mcode
+    // global force T_i^T ef_i
 #pragma unroll
     for (int blk = 0; blk < 6; ++blk)
 #pragma unroll
-        for (int col = 0; col < 3; ++col) {
-            int i = 3 * blk + col;
-            double s = Rc[0][col] * efc[3 * blk] + Rc[1][col] * efc[3 * blk + 1] + Rc[2][col] * efc[3 * blk + 2];
-            int32_t q = mc[i];
-            if (q) f[q - 1] += s;
-        }
+        for (int col = 0; col < 3; ++col)
+            h[e * 18 + 3 * blk + col] =
+                Rc[0][col] * efc[3 * blk] + Rc[1][col] * efc[3 * blk + 1] + Rc[2][col] * efc[3 * blk + 2];
+}
+
+// f += the corner forces of the shells at each joint, one thread per free
+// slot, in colour order (the order of a launch per colour: bitwise the same)
+__global__ void k_shell_forces_gather(const int32_t* __restrict__ jptr, const int32_t* __restrict__ jitem,
+                                      const int32_t* __restrict__ eq, long nslot, int bs,
+                                      const double* __restrict__ h, double* __restrict__ f) {
+    const long r = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (r >= nslot || eq[r] < 0) return;
+    const long j = r / bs;
+    const int s = int(r % bs);
+    if (s >= 6 || jptr[j] == jptr[j + 1]) return;
+    double acc = f[eq[r]];
+    for (int32_t it = jptr[j]; it < jptr[j + 1]; ++it) acc += h[long(jitem[it]) * 6 + s];
+    f[eq[r]] = acc;
 }
 
 // ---------------------------------------------------------------- truss math
@@ -431,15 +446,14 @@ __global__ void k_truss_tangent(const int32_t* __restrict__ els, int n, const in
 // under ANAFLAG 3 (yield non-null) N at or beyond the squash load,
 // (N/Py)^2 >= 1 - tol, is set to +-Py with no plastic strain kept
 // (truss.c:336-347).
-__global__ void k_truss_forces(const int32_t* __restrict__ els, int n, const int32_t* __restrict__ mcode,
-                               const double* __restrict__ c1, const double* __restrict__ c2,
-                               const double* __restrict__ c3, const double* __restrict__ emod,
+// Every bar in one launch; k_truss_forces_gather adds the end forces.
+__global__ void k_truss_forces(int n, const double* __restrict__ emod,
                                const double* __restrict__ carea, const double* __restrict__ llen,
                                const double* __restrict__ defllen, const double* __restrict__ yield,
-                               double* __restrict__ ef_i, double* __restrict__ f) {
+                               double* __restrict__ ef_i) {
     int it = blockIdx.x * blockDim.x + threadIdx.x;
     if (it >= n) return;
-    const long e = els[it];
+    const long e = it;
     const double L0 = llen[e], L = defllen[e];
     const double eps = (L - L0) / L0;
     double N = emod[e] * carea[e] * (eps + 0.5 * (eps * eps)) * L / L0;
@@ -449,11 +463,24 @@ __global__ void k_truss_forces(const int32_t* __restrict__ els, int n, const int
     }
     ef_i[e * 2] = N;
     ef_i[e * 2 + 1] = -N;
-    const double c[3] = {c1[e], c2[e], c3[e]};
-    for (int j = 0; j < 6; ++j) {
-        int32_t q = mcode[e * 6 + j];
-        if (q) f[q - 1] -= ((j < 3) ? N : -N) * c[j % 3];
-    }
+}
+
+// f -= the end forces of the bars at each joint, one thread per free slot, in
+// colour order
+__global__ void k_truss_forces_gather(const int32_t* __restrict__ jptr, const int32_t* __restrict__ jitem,
+                                      const int32_t* __restrict__ eq, long nslot, int bs,
+                                      const double* __restrict__ c1, const double* __restrict__ c2,
+                                      const double* __restrict__ c3, const double* __restrict__ ef_i,
+                                      double* __restrict__ f) {
+    const long r = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (r >= nslot || eq[r] < 0) return;
+    const long j = r / bs;
+    const int s = int(r % bs);
+    if (s >= 3 || jptr[j] == jptr[j + 1]) return;
+    const double* c = s == 0 ? c1 : s == 1 ? c2 : c3;
+    double acc = f[eq[r]];
+    for (int32_t it = jptr[j]; it < jptr[j + 1]; ++it) acc -= ef_i[jitem[it]] * c[jitem[it] >> 1];
+    f[eq[r]] = acc;
 }
 
 // ---------------------------------------------------------------- linear forces
@@ -831,23 +858,20 @@ void launch_forces(Dev& d, int gx, double* f, const double* dd) {
         CB_CHECK(hipGetLastError());
         return;
     }
-    for (size_t c = 0; c + 1 < d.col_ptr_tr.size(); ++c) {
-        int n = d.col_ptr_tr[c + 1] - d.col_ptr_tr[c];
-        if (!n) continue;
-        hipLaunchKernelGGL(k_truss_forces, dim3(nblk(n)), dim3(TPB), 0, d.s,
-                           d.col_el_tr + d.col_ptr_tr[c], n, d.mcode, d.c1[G_I], d.c2[G_I], d.c3[G_I],
-                           d.emod, d.carea, d.llen, d.defllen[G_I], d.anaflag == 3 ? d.yield : nullptr,
-                           d.ef[G_I], f);
+    if (d.ntr) {
+        hipLaunchKernelGGL(k_truss_forces, dim3(nblk(d.ntr)), dim3(TPB), 0, d.s, int(d.ntr), d.emod, d.carea, d.llen,
+                           d.defllen[G_I], d.anaflag == 3 ? d.yield : nullptr, d.ef[G_I]);
+        hipLaunchKernelGGL(k_truss_forces_gather, dim3(nblk(d.nslot)), dim3(TPB), 0, d.s, d.jnt_ptr_tr, d.jnt_item_tr,
+                           d.eq_of_slot, d.nslot, d.bs, d.c1[G_I], d.c2[G_I], d.c3[G_I], d.ef[G_I], f);
     }
     if (d.nfr) launch_frame_forces(d, f, dd);
-    for (size_t c = 0; c + 1 < d.col_ptr_sh.size(); ++c) {
-        int n = d.col_ptr_sh[c + 1] - d.col_ptr_sh[c];
-        if (!n) continue;
-        hipLaunchKernelGGL(k_shell_forces, dim3(nblk(n, 128)), dim3(128), 0, d.s,
-                           d.col_el_sh + d.col_ptr_sh[c], n, d.minc, d.mcode, d.x[gx], dd,
-                           d.c1[G_IP], d.c2[G_IP], d.c3[G_IP], d.c1[G_I], d.c2[G_I], d.c3[G_I],
+    if (d.nsh) {
+        hipLaunchKernelGGL(k_shell_forces, dim3(nblk(d.nsh, 128)), dim3(128), 0, d.s, int(d.nsh), d.minc, d.mcode,
+                           d.x[gx], dd, d.c1[G_IP], d.c2[G_IP], d.c3[G_IP], d.c1[G_I], d.c2[G_I], d.c3[G_I],
                            d.emod, d.nu, d.thick, d.xlocal, d.farea, d.slength, d.ef[G_IP],
-                           d.ef[G_I], f, io, to, po, mo, eo);
+                           d.ef[G_I], d.sh, io, to, po, mo, eo);
+        hipLaunchKernelGGL(k_shell_forces_gather, dim3(nblk(d.nslot)), dim3(TPB), 0, d.s, d.jnt_ptr_sh, d.jnt_item_sh,
+                           d.eq_of_slot, d.nslot, d.bs, d.sh, f);
     }
     CB_CHECK(hipGetLastError());
 }
@@ -980,6 +1004,11 @@ void dev_create(Dev& d, const Model& m) {
     d.gat_item_fr = upi(m.gat_item_fr);
     d.jnt_ptr_fr = upi(m.jnt_ptr_fr);
     d.jnt_item_fr = upi(m.jnt_item_fr);
+    d.jnt_ptr_tr = upi(m.jnt_ptr_tr);
+    d.jnt_item_tr = upi(m.jnt_item_tr);
+    d.jnt_ptr_sh = upi(m.jnt_ptr_sh);
+    d.jnt_item_sh = upi(m.jnt_item_sh);
+    d.sh = dalloc<double>(size_t(m.nsh * 18));
     d.fh = dalloc<double>(size_t(m.nfr * 14));   // 2 bs end forces per member
     d.emod = upd(m.emod);
     d.carea = upd(m.carea);
@@ -1048,7 +1077,8 @@ void dev_reset_state(Dev& d, const Model& m) {
 void dev_destroy(Dev& d) {
     void* ps[] = {d.minc, d.mcode, d.jcode, d.eq_of_slot, d.rowptr, d.colidx, d.diagblk, d.blk_tr,
                   d.blk_sh, d.blk_fr, d.col_el_tr, d.col_el_sh, d.col_el_fr, d.blkrow, d.gat_ptr_fr,
-                  d.gat_item_fr, d.jnt_ptr_fr, d.jnt_item_fr, d.fh, d.emod, d.carea,
+                  d.gat_item_fr, d.jnt_ptr_fr, d.jnt_item_fr, d.fh, d.jnt_ptr_tr, d.jnt_item_tr,
+                  d.jnt_ptr_sh, d.jnt_item_sh, d.sh, d.emod, d.carea,
                   d.llen, d.dens, d.gmod, d.istrong, d.iweak, d.ipolar, d.iwarp, d.auxpt, d.ofs, d.relmask, d.nu,
                   d.thick, d.xlocal, d.farea, d.slength, d.K, d.K32, d.red, d.yield, d.zstrong,
                   d.zweak, d.yld, d.pl_efc, d.pl_tau, d.pl_code, d.pl_st};

@@ -652,16 +652,21 @@ void build_pattern(Model& m) {
     for (int32_t e : m.col_el_fr)
         for (int q = 0; q < 4; ++q)
             m.gat_item_fr[size_t(fill[size_t(m.blk_fr[size_t(e) * 4 + q])]++)] = e * 4 + q;
-    const long fo = m.ntr * 2;
-    m.jnt_ptr_fr.assign(size_t(m.nj) + 1, 0);
-    for (long e = 0; e < m.nfr; ++e)
-        for (int a = 0; a < 2; ++a) m.jnt_ptr_fr[size_t(m.minc[size_t(fo + e * 2 + a)])]++;   // 1-based joint
-    for (long j = 0; j < m.nj; ++j) m.jnt_ptr_fr[size_t(j) + 1] += m.jnt_ptr_fr[size_t(j)];
-    m.jnt_item_fr.assign(size_t(m.nfr * 2), 0);
-    std::vector<int32_t> jf(m.jnt_ptr_fr.begin(), m.jnt_ptr_fr.end() - 1);
-    for (int32_t e : m.col_el_fr)
-        for (int a = 0; a < 2; ++a)
-            m.jnt_item_fr[size_t(jf[size_t(m.minc[size_t(fo + long(e) * 2 + a)] - 1)]++)] = e * 2 + a;
+    // per joint, the element ends at it in colour order
+    auto by_joint = [&](long ne, int nn, long off, const std::vector<int32_t>& order, std::vector<int32_t>& ptr,
+                        std::vector<int32_t>& item) {
+        ptr.assign(size_t(m.nj) + 1, 0);
+        for (long k = 0; k < ne * nn; ++k) ptr[size_t(m.minc[size_t(off + k)])]++;   // 1-based joint
+        for (long j = 0; j < m.nj; ++j) ptr[size_t(j) + 1] += ptr[size_t(j)];
+        item.assign(size_t(ne * nn), 0);
+        std::vector<int32_t> at(ptr.begin(), ptr.end() - 1);
+        for (int32_t e : order)
+            for (int a = 0; a < nn; ++a)
+                item[size_t(at[size_t(m.minc[size_t(off + long(e) * nn + a)] - 1)]++)] = e * nn + a;
+    };
+    by_joint(m.ntr, 2, 0, m.col_el_tr, m.jnt_ptr_tr, m.jnt_item_tr);
+    by_joint(m.nfr, 2, m.ntr * 2, m.col_el_fr, m.jnt_ptr_fr, m.jnt_item_fr);
+    by_joint(m.nsh, 3, m.ntr * 2 + m.nfr * 2, m.col_el_sh, m.jnt_ptr_sh, m.jnt_item_sh);
 }
 
 }  // namespace cb

@@ -58,6 +58,8 @@ struct Model {
     std::vector<int32_t> blkrow, gat_ptr_fr, gat_item_fr;
     // per joint, the frame member ends at it in colour order: item = member * 2 + end
     std::vector<int32_t> jnt_ptr_fr, jnt_item_fr;
+    // the same for bars (bar * 2 + end) and shells (shell * 3 + corner)
+    std::vector<int32_t> jnt_ptr_tr, jnt_item_tr, jnt_ptr_sh, jnt_item_sh;
     long bandwidth = 0;  // max column height of the skyline
 };
 
