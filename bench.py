@@ -72,15 +72,15 @@ def kernel_model(info, sweeps: str = "chain") -> dict:
       diag   : LDL^T of a 64x64 tile (2/3 T^3) + inverse of its unit factor (T^3/3)
       panel  : m tile products of 2 T^3
       update : m(m+1)/2 tile products of 2 T^3
-      column : one fused launch = diag + panel + update of a column (average
-               over the nt launches of a factorization); its time is the launch
-               period (the nt launches of a factorization timed as one span)
+      column : diag + panel + update of a column (average over the nt columns
+               of a factorization, which the fused schedule runs in one launch);
+               its time is the launch's over nt
       sweeps : every off-diagonal factor tile and every Linv tile read once (8 B
                entries), the right-hand side read and the solution written
-      prep   : the sweeps' chain matrices, two tile products of 2 T^3 per
-               tile row; with the look-ahead sweeps also W_I and V_I (one
-               product each) and the two look-ahead bands (two products per
-               sub-diagonal tile each)
+      prep   : the chain matrices, two tile products per tile row; the block
+               sweeps' matrices (look2, look3): per block of four tile rows 16
+               products for the inverse of its 4 x 4 tiles and 40 for each of
+               its two links
     """
     nt = (info.neq + TILE - 1) // TILE
     w = min((info.bandwidth + TILE - 1) // TILE, nt - 1)
@@ -95,20 +95,16 @@ def kernel_model(info, sweeps: str = "chain") -> dict:
         "band_update": ("mfma", 2.0 * t3 * w * (w + 1) / 2, "TFLOP/s"),
         "band_fwd_sweep": ("hbm", float(sweep_bytes), "GB/s"),
         "band_bwd_sweep": ("hbm", float(sweep_bytes), "GB/s"),
-        "band_sweep_prep": ("mfma", 2.0 * t3 * (2 * nt + (2 * nt + 4 * offd if sweeps in ("look2", "look3") else 0)
-                                                + (2 * (offd + nt) if sweeps == "look3" else 0)),
-                            "TFLOP/s"),
+        "band_sweep_prep": ("mfma", 2.0 * t3 * nt * (24 if sweeps in ("look2", "look3") and nt > 4 else 2), "TFLOP/s"),
     }
 
 
-# HBM bytes per launch of the dominant kernels on the default workloads, from
-# two rocprofv3 counter runs each (FETCH_SIZE, then WRITE_SIZE, KiB per
+# HBM bytes per launch of the batch's factor kernel on the default workload,
+# from two rocprofv3 counter runs (FETCH_SIZE, then WRITE_SIZE, KiB per
 # dispatch), scaled by what the same counters read for an elementwise copy of
-# 256 MiB (FETCH_SIZE x 2.000, WRITE_SIZE x 1.000): k_band_column over the
-# interior launches 3000-3099 of the 256x256 panel, k_band_factor_models over
+# 256 MiB (FETCH_SIZE x 2.000, WRITE_SIZE x 1.000): k_band_factor_models over
 # the 13 rounds of 5 time steps of the 512 frames.
 MEASURED_TRAFFIC = {
-    "band_column": (8647.29 * 2.0 + 12001.31) * 1024.0,
     "band_factor_models": (1679014.64 * 2.0 + 3575412.50) * 1024.0,
 }
 TRAFFIC_SOURCE = ("rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE runs, KiB per dispatch scaled by a 256 MiB "
@@ -466,14 +462,12 @@ def main():
                     help="FP64-residual refinement steps per solve of the fp32 path")
     ap.add_argument("--sweeps", default="look2", choices=("chain", "rows", "look2", "look3"),
                     help="band solve sweeps: chain matrices (the library's default), the two-product "
-                         "row step, or both sweeps on the look-ahead system (rows coupled two back; "
-                         "its band formed after each factorization pays back over the ~13 solves "
-                         "of an arc-length increment)")
+                         "row step, or blocks of four tile rows (look2, look3)")
     ap.add_argument("--learned-sizes", default="10,16,24,32",
                     help="held-out panel sizes n (n x n) of --workload learned")
     ap.add_argument("--schedule", default="fused", choices=("fused", "split"),
-                    help="band factorization schedule: one fused launch per tile column, or "
-                         "diag/panel/update launches")
+                    help="band factorization schedule: one fused launch, or diag/panel/update "
+                         "launches per tile column")
     args = ap.parse_args()
     if args.calibrate_copy > 0:
         import torch
