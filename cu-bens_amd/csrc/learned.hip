@@ -970,7 +970,7 @@ double Learned::loss_grad(Dev& d, const double* const* r, const double* const* u
         // messages: dQ = (dE + dA[row]) * (M > 0)
         float* dQ = dtmp_e_;
         hipLaunchKernelGGL(k_msg_bwd, dim3(nblk(ne_ * H)), dim3(TPB), 0, s_, de_, dga_, erow_, mf_[l], dQ, dyb_e_,
-                           ne_ * H);
+                           ne_);
         GemmArgs Mg{};
         Mg.seg[0] = Seg{hb_[l - 1], erow_, H};
         Mg.seg[1] = Seg{hb_[l - 1], ecol_, H};

@@ -41,8 +41,10 @@ def _panel(n, seed=None, **kw):
     return model_file(f"lpanel{n}_{seed}.txt", txt)
 
 
-def test_blocks_loss_and_gradient_match_oracle():
-    with cubens.GpuModel(_panel(4)) as g, cubens.LearnedPrecond(7) as L:
+@pytest.mark.parametrize("n", [4, 3, 15])   # odd sides: edges no multiple of four
+def test_blocks_loss_and_gradient_match_oracle(n):
+    print(f"[learned] n={n}", flush=True)
+    with cubens.GpuModel(_panel(n)) as g, cubens.LearnedPrecond(7) as L:
         p = _params(11)
         L.set_params(p)
         vals = g.tangent(cubens.GEN_BASE, cubens.GEN_BASE)
