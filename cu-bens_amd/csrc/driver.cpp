@@ -31,6 +31,15 @@ struct Timer {
     }
 };
 
+// Where the statistics of a call go, put back when the call ends, by an
+// exception too
+struct StatsScope {
+    RunStats*& at;
+    RunStats* keep;
+    StatsScope(RunStats*& p, RunStats* st) : at(p), keep(p) { p = st; }
+    ~StatsScope() { at = keep; }
+};
+
 }  // namespace
 
 Analysis::Analysis(Model& m, Dev& d, const RunOptions& o) : m_(m), d_(d), o_(o) {
@@ -215,27 +224,20 @@ void Analysis::tangent(int gx, int g) {
 
 int Analysis::tangent_and_factor(int gx, int g, int* det) {
     RunStats tmpst;
-    RunStats* keep = st_;
-    if (!st_) st_ = &tmpst;
+    StatsScope scope(st_, st_ ? st_ : &tmpst);
     tangent(gx, g);
-    int rc = factor_current(det);
-    st_ = keep;
-    return rc;
+    return factor_current(det);
 }
 
 int Analysis::factor_only(int* det) {
     RunStats tmpst;
-    RunStats* keep = st_;
-    if (!st_) st_ = &tmpst;
-    int rc = factor_current(det);
-    st_ = keep;
-    return rc;
+    StatsScope scope(st_, st_ ? st_ : &tmpst);
+    return factor_current(det);
 }
 
 int Analysis::linear_solve(const double* rhs, double* x) {
     RunStats tmpst;
-    RunStats* keep = st_;
-    if (!st_) st_ = &tmpst;
+    StatsScope scope(st_, st_ ? st_ : &tmpst);
     Timer t(&st_->t_solve, d_.s);
     st_->solves++;
     int rc = 0;
@@ -280,12 +282,11 @@ int Analysis::linear_solve(const double* rhs, double* x) {
             if (!(rel <= 10 * o_.krylov_tol)) rc = 3;
         }
     }
-    st_ = keep;
     return rc;
 }
 
 int Analysis::run(RunStats& st) {
-    st_ = &st;
+    StatsScope scope(st_, &st);
     lpf.clear();
     itecnt.clear();
     dpath.clear();
@@ -325,7 +326,6 @@ int Analysis::run(RunStats& st) {
     CB_CHECK(hipStreamSynchronize(d_.s));
     st.t_total = now_s() - t0;
     st.status = rc;
-    st_ = nullptr;
     return rc;
 }
 
