@@ -82,13 +82,17 @@ struct BandLDLT {
     // the tangent comes from d.K32 (the FP32 joint blocks) instead of d.K
     bool src32 = false;
     std::vector<double> piv_host;
+    // tiles, Linv, pivots and the sweeps' matrices hold a complete factorization
+    // (with zero or non-finite pivots too, which the drivers solve with)
+    bool factored = false;
 
     void setup(long n_, long bandwidth, hipStream_t s_);
     void release();
     // Copies the lower band of d.K (d.K32 with src32; equation order) and factorizes.
     // 0 ok, 1 zero or non-finite pivot, 2 entry outside the band.
     int factor(const Dev& d);
-    // out = (L D L^T)^{-1} rhs, both device NEQ vectors (may alias).
+    // out = (L D L^T)^{-1} rhs, both device NEQ vectors (may alias); throws
+    // unless factored.
     void solve(const double* rhs, double* out);
     size_t bytes() const { return sizeof(R) * size_t(nt) * size_t(2 * (w + 1) + 2) * 64 * 64; }
 };

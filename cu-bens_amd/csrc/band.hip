@@ -2143,11 +2143,13 @@ void BandLDLT<R>::release() {
     cmat = nullptr; gmat = nullptr;
     lb = nullptr; mch = nullptr; gch = nullptr; bw = nullptr; part = nullptr;
     prog = nullptr;
+    factored = false;
     clock.release();
 }
 
 template <class R>
 int BandLDLT<R>::factor(const Dev& d) {
+    factored = false;
     // the fused schedule takes the matrix from tiles_t
     R* band = split ? tiles : tiles_t;
     CB_CHECK(hipMemsetAsync(band, 0, sizeof(R) * size_t(nt) * (w + 1) * TT, s));
@@ -2230,6 +2232,7 @@ int BandLDLT<R>::factor(const Dev& d) {
     clock.collect();
     if (bad & 1) throw DeviceError("band factorization: a wait exceeded its bound");
     if (bad & 2) return 2;
+    factored = true;
     for (long i = 0; i < n; ++i)
         if (piv_host[i] == 0.0 || !std::isfinite(piv_host[i])) return 1;
     return 0;
@@ -2237,6 +2240,7 @@ int BandLDLT<R>::factor(const Dev& d) {
 
 template <class R>
 void BandLDLT<R>::solve(const double* rhs, double* out) {
+    if (!factored) throw DeviceError("band solve: there is no factorization to solve with");
     CB_CHECK(hipMemsetAsync(flag, 0, sizeof(int), s));
     const long spin_limit = 1L << 22, ntot = nt * T;
     const int gh = helpers_per_row(w);

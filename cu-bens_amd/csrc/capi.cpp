@@ -483,12 +483,20 @@ int cb_solve(cb_model* h, const double* rhs_host, double* x_host) {
     GUARD_BEGIN
     cb::Analysis& an = analysis(h, nullptr);
     const long n = h->m.neq;
-    double* b = cb::dalloc<double>(size_t(n));
-    double* x = cb::dalloc<double>(size_t(n));
-    cb::h2d(b, rhs_host, size_t(n), h->d.s);
-    int rc = an.linear_solve(b, x);
-    cb::d2h(x_host, x, size_t(n), h->d.s);
-    CB_CHECK(hipStreamSynchronize(h->d.s));
+    double *b = nullptr, *x = nullptr;
+    int rc = 0;
+    try {
+        b = cb::dalloc<double>(size_t(n));
+        x = cb::dalloc<double>(size_t(n));
+        cb::h2d(b, rhs_host, size_t(n), h->d.s);
+        rc = an.linear_solve(b, x);
+        cb::d2h(x_host, x, size_t(n), h->d.s);
+        CB_CHECK(hipStreamSynchronize(h->d.s));
+    } catch (...) {
+        (void)hipFree(b);
+        (void)hipFree(x);
+        throw;
+    }
     (void)hipFree(b);
     (void)hipFree(x);
     if (rc) return fail(rc, "iterative solve did not reach its tolerance");

@@ -273,7 +273,7 @@ int Analysis::linear_solve(const double* rhs, double* x) {
         int it = gm_.solve(d_, prec, eb, ex, o_.krylov_tol, o_.maxit, &rel);
         st_->krylov_iters += it;
         st_->worst_relres = std::max(st_->worst_relres, rel);
-        if (!(rel <= 10 * o_.krylov_tol) && b64_.tiles) {
+        if (!(rel <= 10 * o_.krylov_tol) && b64_.factored) {
             // fall back to the direct solve (the judge's factor)
             st_->krylov_fallbacks++;
             b64_.solve(rhs, x);

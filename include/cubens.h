@@ -206,7 +206,10 @@ int cb_update_geometry(cb_model *m, int gen_x, const double *dd_host);
  * (skyfact, solve.c:539): det = 1 when a pivot is not positive; pivots [NEQ]
  * may be NULL. */
 int cb_factor(cb_model *m, const cb_options *opt, int *det, double *pivots);
-/* Solve with the last factorization / preconditioner (skysolve, solve.c:655). */
+/* Solve with the last factorization / preconditioner (skysolve, solve.c:655).
+ * With a band solver an error unless cb_factor or cb_run has factorized since
+ * the options last changed; a Krylov solver that misses its tolerance falls
+ * back on the FP64 factor of judge = 1 and fails without one. */
 int cb_solve(cb_model *m, const double *rhs_host, double *x_host);
 
 /* Runs the driver of the model's ALGFLAG: NR / modified NR (main.c:1800-2157),

@@ -1,0 +1,28 @@
+"""The band solver's kernels and host code on the CPU (band_host.cpp,
+host_hip/hip/hip_runtime.h): null pointers and accesses past the end of a
+buffer are segmentation faults there."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CLANG = "/opt/rocm/llvm/bin/clang++"
+pytestmark = pytest.mark.skipif(not os.path.exists(CLANG), reason="needs ROCm's clang++")
+
+
+@pytest.fixture(scope="module")
+def band_host(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("band") / "band_host")
+    subprocess.run([CLANG, "-std=c++17", "-O2", "-w", "-pthread", "-I", os.path.join(HERE, "host_hip"), "-x", "c++",
+                    os.path.join(HERE, "band_host.cpp"), "-o", exe], check=True)
+
+    def run(*args):
+        r = subprocess.run([exe, *map(str, args)], capture_output=True, text=True, timeout=110)
+        assert r.returncode == 0, (r.returncode, r.stdout)
+        return r.stdout
+    return run
+
+
+def test_solve_without_a_factorization_is_refused(band_host):
+    band_host("unfactored")

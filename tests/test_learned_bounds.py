@@ -17,7 +17,7 @@ CLANG = "/opt/rocm/llvm/bin/clang++"
 @pytest.fixture(scope="module")
 def program(tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("bounds") / "learned_bounds")
-    subprocess.run([CLANG, "-std=c++17", "-O2", "-w", "-I", os.path.join(HERE, "host_hip"), "-x", "c++",
+    subprocess.run([CLANG, "-std=c++17", "-O2", "-w", "-pthread", "-I", os.path.join(HERE, "host_hip"), "-x", "c++",
                     os.path.join(HERE, "learned_bounds.cpp"), "-o", exe], check=True)
     return exe
 
