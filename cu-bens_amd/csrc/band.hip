@@ -2196,11 +2196,13 @@ int BandLDLT<R>::factor(const Dev& d) {
         }
     }
     CB_CHECK(hipGetLastError());
+    // each by itself: one that fails leaves the others for the next factorization
+    auto need = [](auto*& p, long count) {
+        if (!p) p = dalloc<std::remove_reference_t<decltype(*p)>>(size_t(count));
+    };
     if (chained && !blocked()) {
-        if (!cmat) {
-            cmat = dalloc<R>(size_t(nt) * TT);
-            gmat = dalloc<R>(size_t(nt) * TT);
-        }
+        need(cmat, nt * TT);
+        need(gmat, nt * TT);
         const bool tk_prep = clock.take(KT_PREP);
         if (tk_prep) clock.begin(KT_PREP, s);
         hipLaunchKernelGGL((k_sweep_chain<R>), dim3(int(nt)), dim3(256), 0, s, tiles, linv, cmat, gmat, nt, w);
@@ -2211,13 +2213,11 @@ int BandLDLT<R>::factor(const Dev& d) {
         const bool tk_prep = clock.take(KT_PREP);
         if (tk_prep) clock.begin(KT_PREP, s);
         const long nb = (nt + SB - 1) / SB;
-        if (!lb) {
-            lb = dalloc<R>(size_t(nb) * LB * TT);
-            mch = dalloc<R>(size_t(nt) * SB * TT);
-            gch = dalloc<R>(size_t(nt) * SB * TT);
-            bw = dalloc<double>(size_t(nt) * T);
-            part = dalloc<double>(size_t(2 * nt * helpers_per_row(w) * T));
-        }
+        need(lb, nb * LB * TT);
+        need(mch, nt * SB * TT);
+        need(gch, nt * SB * TT);
+        need(bw, nt * T);
+        need(part, 2 * nt * helpers_per_row(w) * T);
         hipLaunchKernelGGL((k_block_inverse<R>), dim3(unsigned(nb * (SB - 1))), dim3(NTH), 0, s, tiles, linv, lb, nt,
                            w);
         hipLaunchKernelGGL((k_block_link<R>), dim3(unsigned(2 * nt * SB)), dim3(NTH), 0, s, tiles, tiles_t, linv, lb,

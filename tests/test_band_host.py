@@ -26,3 +26,8 @@ def band_host(tmp_path_factory):
 
 def test_solve_without_a_factorization_is_refused(band_host):
     band_host("unfactored")
+
+
+def test_factorization_recovers_from_each_failed_allocation(band_host):
+    out = band_host("memory")
+    assert "look 0: 2 allocations" in out and "look 2: 5 allocations" in out
