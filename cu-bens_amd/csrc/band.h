@@ -74,7 +74,7 @@ struct BandLDLT {
     double* part = nullptr;
     double* xw = nullptr;    // work vectors (padded)
     double* yw = nullptr;
-    int* flag = nullptr;       // error bits: 1 a wait bound hit, 2 an entry outside the band
+    int* flag = nullptr;       // error bits: 1 a wait bound hit, 2 an entry outside the band; then start counters
     int* prog = nullptr;       // progress counters of the fused factorization launch
     // factorization schedule: one launch for all columns (default), or
     // separate diag/panel/update launches per column
@@ -82,6 +82,8 @@ struct BandLDLT {
     // the tangent comes from d.K32 (the FP32 joint blocks) instead of d.K
     bool src32 = false;
     std::vector<double> piv_host;
+    long spin_limit = 1L << 22;   // polls of a wait before it counts as failed
+    int counted = 1024;           // workgroups up to which a launch numbers them by count (start_number)
     // tiles, Linv, pivots and the sweeps' matrices hold a complete factorization
     // (with zero or non-finite pivots too, which the drivers solve with)
     bool factored = false;

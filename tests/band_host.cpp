@@ -3,6 +3,8 @@
 // with one slot per joint.
 //   band_host solve n b [xcds slots]   fused and split factors bitwise equal, each
 //                                      sweep schedule solves the system, FP64 and FP32
+//   band_host pair n b xcds slots [counted]  two handles at once: their factorizations
+//                                      and solves, each the result of a handle alone
 //   band_host unfactored               a solve without a factor is an error
 //   band_host memory                   a factorization whose k-th allocation fails,
 //                                      for every k, is an error and can be repeated
@@ -101,6 +103,55 @@ template <class R> int solve_all(long n, long b, double eps) {
     return 0;
 }
 
+// Two handles' launches, the i-th of one beside the i-th of the other
+template <class F> void side_by_side(F&& a, F&& b) {
+    std::vector<host_hip::Launch> la, lb;
+    host_hip::held = &la;
+    a();
+    host_hip::held = &lb;
+    b();
+    host_hip::held = nullptr;
+    for (size_t i = 0; i < la.size(); ++i) host_hip::run({la[i], lb[i]});
+}
+
+int pair(long n, long b, int xcds, int slots, int counted) {
+    Problem p(n, b);
+    BandLDLT<double> alone, two[2];
+    for (int sweeps = 0; sweeps < 3; ++sweeps) {
+        auto prepare = [&](BandLDLT<double>& f) {
+            f.setup(n, b, nullptr);
+            f.chained = sweeps != 1;
+            f.look = sweeps == 2 ? 2 : 0;
+            f.spin_limit = 200000;
+            f.counted = counted;
+        };
+        for (BandLDLT<double>* f : {&alone, &two[0], &two[1]}) prepare(*f);
+        host_hip::xcds = 4;
+        host_hip::slots = 2;
+        if (alone.factor(p.d) != 0 || !(p.solve(alone) < 1e-14)) return 1;
+        std::vector<double> x(static_cast<size_t>(n), 1.0);
+        double *rhs = nullptr, *out = cb::dalloc<double>(x.size());
+        Problem::up(rhs, x);
+        alone.solve(rhs, out);
+        host_hip::xcds = xcds;
+        host_hip::slots = slots;
+        auto factor = [&](int i) { return [&, i] { two[i].factor(p.d); }; };
+        auto solve = [&](int i) { return [&, i] { two[i].solve(rhs, out); }; };
+        side_by_side<std::function<void()>>(factor(0), factor(1));
+        const int bad = two[0].flag[0] | two[1].flag[0];
+        std::printf("sweeps %d: factorizations %s\n", sweeps, bad ? "stopped at a wait's bound" : "ended");
+        if (bad) return 1;
+        side_by_side<std::function<void()>>(solve(0), solve(1));
+        const int bad2 = two[0].flag[0] | two[1].flag[0];
+        std::printf("sweeps %d: solves %s\n", sweeps, bad2 ? "stopped at a wait's bound" : "ended");
+        if (bad2) return 1;
+        for (BandLDLT<double>& f : two)
+            if (!same(f.piv, alone.piv, size_t(n)) || !same(f.xw, alone.xw, size_t(n)))
+                return std::printf("the results differ from a handle's alone\n"), 1;
+    }
+    return 0;
+}
+
 template <class F> bool refused(F&& call) {
     try {
         call();
@@ -122,6 +173,7 @@ int main(int argc, char** argv) {
         // 64-term sums of products, a few hundred of them after one another
         return solve_all<double>(n, b, 1e-14) || solve_all<float>(n, b, 1e-6);
     }
+    if (what == "pair") return pair(arg(2, 600), arg(3, 200), int(arg(4, 4)), int(arg(5, 2)), int(arg(6, 1024)));
     if (what == "unfactored") {
         Problem p(400, 70);
         for (int sweeps = 0; sweeps < 3; ++sweeps) {

@@ -132,6 +132,10 @@ inline void block_barrier() {
     ++f.blocks;
     while (block_here < long(fibers.size()) * f.blocks) yield();
 }
+inline void wait_stores() {   // the stores of the whole wavefront
+    wave_barrier();
+    std::atomic_thread_fence(std::memory_order_seq_cst);
+}
 inline void poll_pause() {
     if (self % 64 == 0) sched_yield();
     yield();
@@ -271,7 +275,7 @@ inline int atomicOr(int* p, int v) { return __atomic_fetch_or(p, v, __ATOMIC_SEQ
 #define __builtin_amdgcn_readfirstlane host_hip::readfirstlane
 #define __builtin_amdgcn_wave_barrier host_hip::wave_barrier
 #define __builtin_amdgcn_s_sleep(n) host_hip::poll_pause()
-#define __builtin_amdgcn_s_waitcnt(n) std::atomic_thread_fence(std::memory_order_seq_cst)
+#define __builtin_amdgcn_s_waitcnt(n) host_hip::wait_stores()
 #define __builtin_amdgcn_rcp(x) (1.0 / (x))
 #define __builtin_amdgcn_make_buffer_rsrc(p, stride, n, flags) host_hip::Buffer{reinterpret_cast<char*>(p), size_t(n)}
 #define __builtin_amdgcn_raw_buffer_store_b128(v, b, off, soff, aux) host_hip::buffer_store(v, b, size_t(off))

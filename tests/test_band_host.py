@@ -31,3 +31,14 @@ def test_solve_without_a_factorization_is_refused(band_host):
 def test_factorization_recovers_from_each_failed_allocation(band_host):
     out = band_host("memory")
     assert "look 0: 2 allocations" in out and "look 2: 5 allocations" in out
+
+
+# (equations, half-bandwidth, XCDs, workgroups at once on each, launches
+# numbered by count up to): the dispatch starts one launch's workgroups first
+# on every other XCD, so that workgroups that wait for others in index order
+# fill both XCDs and never end
+@pytest.mark.parametrize("n,b,xcds,slots,counted", [(600, 200, 4, 2, 1024), (600, 200, 2, 3, 1024), (700, 40, 4, 2, 1024),
+                                                    (1000, 640, 4, 3, 1024), (2600, 300, 8, 8, 16)])
+def test_two_handles_at_once(band_host, n, b, xcds, slots, counted):
+    out = band_host("pair", n, b, xcds, slots, counted)
+    assert out.count("ended") == 6
