@@ -83,7 +83,18 @@ struct BandLDLT {
     bool src32 = false;
     std::vector<double> piv_host;
     long spin_limit = 1L << 22;   // polls of a wait before it counts as failed
-    int counted = 1024;           // workgroups up to which a launch numbers them by count (start_number)
+    // Whether a factorization or row sweep numbers its workgroups by count
+    // (band.hip, start_number): one atomic instead of four accesses after one
+    // another, and consecutive rows lie close to each other.  Against blockIdx.x
+    // row sweeps of 57, 195, 390 and 892 tile rows (3 to 10 tiles below the
+    // diagonal) take 0.95, 0.90, 0.95 and 1.01 of the time by count and 1.02,
+    // 1.00, 1.04 and 1.03 by index; 2426 and 6168 rows 1.04 and 1.06 by count,
+    // 1.02 and 1.01 by index; 221, 390 and 608 rows of a full matrix 1.00, 1.20
+    // and 1.24 by count, where whole XCDs stream at once, and 1.10, 1.08 and
+    // 1.05 by index.  The factorization of 6168 columns: 18.0 us a column by
+    // count, 17.7 by index and by blockIdx.x.
+    int counted = 1024;   // workgroups
+    bool by_count(long workgroups) const { return workgroups <= counted && w <= 256; }
     // tiles, Linv, pivots and the sweeps' matrices hold a complete factorization
     // (with zero or non-finite pivots too, which the drivers solve with)
     bool factored = false;

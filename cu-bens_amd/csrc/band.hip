@@ -141,14 +141,20 @@ __device__ __forceinline__ long start_by_count(int* counter) {
 // workgroup takes its own number once that is less than AHEAD past the count
 // of the numbers taken.  While one XCD cannot start its workgroups, the other
 // seven so take at most 7 AHEAD numbers past the lowest free one.  The rest
-// of the workgroups hold back, and after PATIENCE polls (about 1 ms; a launch
-// that has the GPU to itself holds back for some ten us at its start) take
-// the lowest free number, as does one whose own number was taken like that.
+// of the workgroups hold back, and after PATIENCE polls (about 8 ms) take the
+// lowest free number, as does one whose own number was taken like that.  A
+// launch that has the GPU to itself holds back too, for some ten us at its
+// start and while one XCD is behind the others: with a patience of 1024 polls
+// a full matrix of 390 and 608 tile rows took 1.12 and 1.4 times as long to
+// factor, from 4096 on no longer than by blockIdx.x.
 // So some workgroup can go on as long as the GPU has room for 7 AHEAD
 // workgroups of every such launch at once.
+// Not for launches of many short workgroups: the block sweeps, whose helpers
+// live for some ten us, take seven times as long (388 tiles below the
+// diagonal).
 // counter[0] is the count, counter[1 ..] the numbers taken, a bit each, zero
 // before the launch.
-constexpr int AHEAD = 8, PATIENCE = 1 << 10;
+constexpr int AHEAD = 8, PATIENCE = 1 << 13;
 __device__ __forceinline__ long start_by_index(int* counter) {
     __shared__ int number;
     if (threadIdx.x == 0) {
@@ -177,15 +183,8 @@ __device__ __forceinline__ long start_by_index(int* counter) {
     return __builtin_amdgcn_readfirstlane(number);
 }
 
-// Launches of up to `counted` workgroups (BandLDLT) go by count, one atomic
-// instead of four accesses after one another; most of their workgroups start at
-// once.  Measured against blockIdx.x, forward / backward row sweeps of 57, 900,
-// 2426 and 6168 tile rows: by count 53 / 54 us (from 55.5 / 56), 982 / 1016
-// (980 / 1002), 2510 / 2690 (2430 / 2550), 6400 / 6900 (6150 / 6420); by index
-// 57 / 58, 1010 / 1045, 2460 / 2590, 6180 / 6495.  The factorization of 6168
-// columns: 18.0 us a column by count, 17.7 by index and by blockIdx.x.
-__device__ __forceinline__ long start_number(int* counter, int counted) {
-    return int(gridDim.x) <= counted ? start_by_count(counter) : start_by_index(counter);
+__device__ __forceinline__ long start_number(int* counter, bool by_count) {
+    return by_count ? start_by_count(counter) : start_by_index(counter);
 }
 
 __device__ __forceinline__ double lane_value(double x, int lane) {
@@ -771,7 +770,7 @@ inline long factor_workgroups(long nt, int w) {
 template <class R>
 __global__ void __launch_bounds__(NTH) k_band_factor(R* __restrict__ tiles, R* __restrict__ tiles_t,
                                                      R* __restrict__ linv, double* __restrict__ piv, int w, long nt,
-                                                     int* prog, int* started, int counted, long spin_limit,
+                                                     int* prog, int* started, bool by_count, long spin_limit,
                                                      int* err) {
     constexpr int N = TileAcc<R>::N, NS = TT / NTH;
     __shared__ R xs[T][T];
@@ -831,7 +830,7 @@ __global__ void __launch_bounds__(NTH) k_band_factor(R* __restrict__ tiles, R* _
         stage<true>(ys, linv + K * (long)TT);
     };
 
-    const long number = gridDim.x > 1 ? start_number(started, counted) : 0;
+    const long number = gridDim.x > 1 ? start_number(started, by_count) : 0;
     if (number == 0) {
         if (tid < 2) drained_s[tid] = 0;
         // A column's tiles sit in the pair (a0, a1): A_{J,J-1} and Linv_{J-1},
@@ -1213,11 +1212,11 @@ __device__ __forceinline__ void put_value(double* p, double x) {
 template <class R>
 __global__ void __launch_bounds__(256) k_fwd_sweep(const R* __restrict__ tiles, const R* __restrict__ linv,
                                                    double* __restrict__ xr, double* y, long nt, int w,
-                                                   int* started, int counted, long spin_limit, int* err) {
+                                                   int* started, bool by_count, long spin_limit, int* err) {
     __shared__ double vin[T];
     __shared__ double vch[NCH][T];
     __shared__ double part[4][T];
-    const long I = start_number(started, counted);
+    const long I = start_number(started, by_count);
     const int tid = threadIdx.x, row = tid % T, q = tid / T, k0 = 16 * q;
     R lv[16], ln[16];
     const R* lvp = linv + I * (long)TT;
@@ -1280,11 +1279,12 @@ __global__ void __launch_bounds__(256) k_fwd_sweep(const R* __restrict__ tiles, 
 template <class R>
 __global__ void __launch_bounds__(256) k_bwd_sweep(const R* __restrict__ tiles_t, const R* __restrict__ linv,
                                                    const double* __restrict__ y, const double* __restrict__ piv,
-                                                   double* x, long nt, int w, int* started, int counted, long spin_limit, int* err) {
+                                                   double* x, long nt, int w, int* started, bool by_count,
+                                                   long spin_limit, int* err) {
     __shared__ double vin[T];
     __shared__ double vch[NCH][T];
     __shared__ double part[4][T];
-    const long I = nt - 1 - start_number(started, counted);
+    const long I = nt - 1 - start_number(started, by_count);
     const int tid = threadIdx.x, col = tid % T, q = tid / T, k0 = 16 * q;
     R lv[16], ln[16];
     const R* lvp = linv + I * (long)TT;
@@ -1395,11 +1395,11 @@ __global__ void __launch_bounds__(256) k_sweep_chain(const R* __restrict__ tiles
 template <class R>
 __global__ void __launch_bounds__(256) k_fwd_sweep_m(const R* __restrict__ tiles, const R* __restrict__ linv,
                                                      const R* __restrict__ mch, double* __restrict__ xr, double* y,
-                                                     long nt, int w, int* started, int counted, long spin_limit, int* err) {
+                                                     long nt, int w, int* started, bool by_count, long spin_limit, int* err) {
     __shared__ double vin[T];
     __shared__ double vch[NCH][T];
     __shared__ double part[4][T];
-    const long I = start_number(started, counted);
+    const long I = start_number(started, by_count);
     const int tid = threadIdx.x, row = tid % T, q = tid / T, k0 = 16 * q;
     R lv[16], lm[16];
     const R* lvp = linv + I * (long)TT;
@@ -1466,11 +1466,11 @@ template <class R>
 __global__ void __launch_bounds__(256) k_bwd_sweep_m(const R* __restrict__ tiles_t, const R* __restrict__ linv,
                                                      const R* __restrict__ gch, const double* __restrict__ y,
                                                      const double* __restrict__ piv, double* x, long nt, int w,
-                                                     int* started, int counted, long spin_limit, int* err) {
+                                                     int* started, bool by_count, long spin_limit, int* err) {
     __shared__ double vin[T];
     __shared__ double vch[NCH][T];
     __shared__ double part[4][T];
-    const long I = nt - 1 - start_number(started, counted);
+    const long I = nt - 1 - start_number(started, by_count);
     const int tid = threadIdx.x, col = tid % T, q = tid / T, k0 = 16 * q;
     R lv[16], lm[16];
     const R* lvp = linv + I * (long)TT;
@@ -2249,7 +2249,7 @@ int BandLDLT<R>::factor(const Dev& d) {
             clock.begin(KT_COLUMN, s, nt);
         }
         hipLaunchKernelGGL((k_band_factor<R>), dim3(unsigned(grid)), dim3(NTH), 0, s, tiles,
-                           tiles_t, linv, piv, w, nt, prog, prog + P_N * nt * PSTRIDE, counted, spin_limit, flag);
+                           tiles_t, linv, piv, w, nt, prog, prog + P_N * nt * PSTRIDE, by_count(grid), spin_limit, flag);
         if (tk_column) clock.end(s);
     } else {
         for (long Kt = 0; Kt < nt; ++Kt) {
@@ -2335,10 +2335,10 @@ void BandLDLT<R>::solve(const double* rhs, double* out) {
                            part, nt, w, gh, flag + PSTRIDE, spin_limit, flag);
     else if (chained)
         hipLaunchKernelGGL((k_fwd_sweep_m<R>), dim3(int(nt)), dim3(256), 0, s, tiles, linv, cmat, xw, yw, nt, w,
-                           flag + PSTRIDE, counted, spin_limit, flag);
+                           flag + PSTRIDE, by_count(nt), spin_limit, flag);
     else
         hipLaunchKernelGGL((k_fwd_sweep<R>), dim3(int(nt)), dim3(256), 0, s, tiles, linv, xw, yw, nt, w,
-                           flag + PSTRIDE, counted, spin_limit, flag);
+                           flag + PSTRIDE, by_count(nt), spin_limit, flag);
     if (tk_fwd) clock.end(s);
     const bool tk_bwd = clock.take(KT_BWD);
     if (tk_bwd) clock.begin(KT_BWD, s);
@@ -2347,10 +2347,10 @@ void BandLDLT<R>::solve(const double* rhs, double* out) {
                            part + npart, nt, w, gh, flag + PSTRIDE + start_counters(nt), spin_limit, flag);
     else if (chained)
         hipLaunchKernelGGL((k_bwd_sweep_m<R>), dim3(int(nt)), dim3(256), 0, s, tiles_t, linv, gmat, yw, piv, xw, nt, w,
-                           flag + PSTRIDE + start_counters(nt), counted, spin_limit, flag);
+                           flag + PSTRIDE + start_counters(nt), by_count(nt), spin_limit, flag);
     else
         hipLaunchKernelGGL((k_bwd_sweep<R>), dim3(int(nt)), dim3(256), 0, s, tiles_t, linv, yw, piv, xw, nt, w,
-                           flag + PSTRIDE + start_counters(nt), counted, spin_limit, flag);
+                           flag + PSTRIDE + start_counters(nt), by_count(nt), spin_limit, flag);
     if (tk_bwd) clock.end(s);
     CB_CHECK(hipGetLastError());
     CB_CHECK(hipMemcpyAsync(out, xw, sizeof(double) * size_t(n), hipMemcpyDeviceToDevice, s));
