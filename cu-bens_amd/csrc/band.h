@@ -11,13 +11,13 @@ namespace cb {
 // Kernel families of the band solver whose launches can be timed with HIP
 // events: KT_COLUMN is the fused factorization, per tile column; KT_DIAG,
 // KT_PANEL and KT_UPDATE are the launches of the split schedule.
-// KT_PREP times the launches that form the sweeps' block matrices after a
-// factorization.
+// KT_PREP times the launches that form the sweeps' matrices (chain matrices,
+// or block inverses and links) after a factorization.
 enum { KT_COLUMN = 0, KT_DIAG = 1, KT_PANEL = 2, KT_UPDATE = 3, KT_FWD = 4, KT_BWD = 5, KT_PREP = 6, KT_N = 7 };
 
 // Launches of a selected family are bracketed by two events.  The fused
-// factorization is one launch and counts as its nt tile columns; of the split schedule's launches only every `every`-th is timed;
-// the sweeps are always timed.  launches counts every launch issued and ms is
+// factorization is one launch and counts as its nt tile columns; of the split
+// schedule's launches only every `every`-th is timed; the sweeps are always timed.  launches counts every launch issued and ms is
 // the timed total scaled to all of them, so ms / launches is the average
 // launch duration.
 struct KernelClock {
@@ -61,8 +61,8 @@ struct BandLDLT {
     // right-hand side [nt * 64] and the helpers' partial sums; allocated at the
     // first factorization that needs them
     bool chained = true;     // sweeps with formed matrices, or the two-product row step
-    int look = 0;            // with chained: 2 or 3, the block sweeps
-    bool blocked() const { return chained && look >= 2 && nt > 4; }
+    bool blocks = false;     // with chained: the block sweeps, where there is more than one block
+    bool blocked() const { return chained && blocks && nt > 4; }
     // otherwise the chain matrices M_I = Linv_I L_{I,I-1} and G_I = L_{I+1,I}
     // Linv_I, [nt] tiles each, allocated at the first factorization too
     R* cmat = nullptr;

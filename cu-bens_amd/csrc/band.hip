@@ -8,13 +8,14 @@
 //
 // Storage: the lower band (half-bandwidth b = max column height) in dense T x T
 // tiles; tile row I holds tiles J = I-w .. I (w = ceil(b/T)), column-major.
-// Factorization is right-looking by tile column K:
-//   diag : D_K and Linv_K = L_KK^{-1} of A_KK = L_KK D_K L_KK^T, in registers
+// Factorization by tile tasks of column K (left-looking in one launch, or
+// right-looking with a launch per kind of task):
+//   diag : D_K and Linv_K = L_KK^{-1} of A_KK = L_KK D_K L_KK^T, in LDS
 //   panel: L_IK = A_IK Linv_K^T D_K^{-1},            K < I <= K+w
 //   update: A_IJ -= (L_IK D_K) L_JK^T,               K < J <= I <= K+w
-// Solves: pipelined forward and backward sweeps, one workgroup per tile row,
-// with Linv_I for the diagonal blocks and pivot scaling folded into the
-// backward sweep.
+// Solves: pipelined forward and backward sweeps, one workgroup per tile row or
+// several per block of four, with Linv_I for the diagonal blocks and pivot
+// scaling folded into the backward sweep.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -100,8 +100,9 @@ enum { CB_FACTOR_FUSED = 0, CB_FACTOR_SPLIT = 1 };
  * (CB_SWEEP_CHAIN, the default), or of two dependent 64x64 products
  * (CB_SWEEP_ROWS), or blocks of four tile rows, with the block inverses and the
  * links between neighbouring blocks formed after each factorization
- * (CB_SWEEP_LOOK2 and CB_SWEEP_LOOK3, which named look-ahead systems before):
- * less than half the time per solve. */
+ * (CB_SWEEP_LOOK2; CB_SWEEP_LOOK3 is another name for it): less than half the
+ * time per solve from some hundred tile rows on.  Models of up to four tile
+ * rows take the chain matrices. */
 enum { CB_SWEEP_CHAIN = 0, CB_SWEEP_ROWS = 1, CB_SWEEP_LOOK2 = 2, CB_SWEEP_LOOK3 = 3 };
 
 /* Generations of the per-element state (base = last converged, _i = current
@@ -112,7 +113,7 @@ enum { CB_GEN_BASE = 0, CB_GEN_I = 1, CB_GEN_IP = 2 };
 /* Kernel families of the band solver (timed with HIP events on their stream):
  * the fused factorization launch (per tile column), the diag/panel/update launches
  * of the split schedule, the forward and backward sweeps, and the launches
- * that form the sweeps' block matrices after a factorization. */
+ * that form the sweeps' matrices after a factorization. */
 enum { CB_KT_COLUMN = 0, CB_KT_DIAG = 1, CB_KT_PANEL = 2, CB_KT_UPDATE = 3, CB_KT_FWD = 4, CB_KT_BWD = 5,
        CB_KT_PREP = 6, CB_KT_N = 7 };
 

@@ -85,7 +85,7 @@ template <class R> int solve_all(long n, long b, double eps) {
     std::printf("%ld equations, %ld tile rows, %d tiles below the diagonal\n", n, f.nt, f.w);
     for (int sweeps = 0; sweeps < 3; ++sweeps) {
         f.chained = sweeps != 1;
-        f.look = sweeps == 2 ? 2 : 0;
+        f.blocks = sweeps == 2;
         if (f.factor(p.d) != 0) return std::printf("fused schedule: not factored\n"), 1;
         for (long I = 0; I < f.nt; ++I) {
             bool ok = same(f.linv + I * cb::TT, split.linv + I * cb::TT, cb::TT) &&
@@ -121,7 +121,7 @@ int pair(long n, long b, int xcds, int slots, int counted) {
         auto prepare = [&](BandLDLT<double>& f) {
             f.setup(n, b, nullptr);
             f.chained = sweeps != 1;
-            f.look = sweeps == 2 ? 2 : 0;
+            f.blocks = sweeps == 2;
             f.spin_limit = 200000;
             f.counted = counted;
         };
@@ -179,7 +179,7 @@ int main(int argc, char** argv) {
         for (int sweeps = 0; sweeps < 3; ++sweeps) {
             BandLDLT<double> f;
             f.chained = sweeps != 1;
-            f.look = sweeps == 2 ? 2 : 0;
+            f.blocks = sweeps == 2;
             f.setup(p.n, p.b, nullptr);
             if (!refused([&] { p.solve(f); })) return 1;
             if (f.factor(p.d) != 0 || !(p.solve(f) < 1e-14)) return 1;
@@ -190,11 +190,11 @@ int main(int argc, char** argv) {
     }
     if (what == "memory") {
         Problem p(400, 70);
-        for (int look = 0; look < 3; look += 2) {
+        for (bool blocks : {false, true}) {
             int failures = 0;
             for (long k = 0;; ++k) {
                 BandLDLT<double> f;
-                f.look = look;
+                f.blocks = blocks;
                 f.setup(p.n, p.b, nullptr);
                 host_hip::fail_at = k;
                 const bool failed = [&] {
@@ -211,7 +211,7 @@ int main(int argc, char** argv) {
                 if (!refused([&] { p.solve(f); })) return 1;
                 if (f.factor(p.d) != 0 || !(p.solve(f) < 1e-14)) return 1;
             }
-            std::printf("look %d: %d allocations, each failed once\n", look, failures);
+            std::printf("%s sweeps: %d allocations, each failed once\n", blocks ? "block" : "chain", failures);
             if (!failures) return 1;
         }
         return 0;

@@ -30,7 +30,7 @@ def test_solve_without_a_factorization_is_refused(band_host):
 
 def test_factorization_recovers_from_each_failed_allocation(band_host):
     out = band_host("memory")
-    assert "look 0: 2 allocations" in out and "look 2: 5 allocations" in out
+    assert "chain sweeps: 2 allocations" in out and "block sweeps: 5 allocations" in out
 
 
 # (equations, half-bandwidth, XCDs, workgroups at once on each, launches
@@ -42,3 +42,10 @@ def test_factorization_recovers_from_each_failed_allocation(band_host):
 def test_two_handles_at_once(band_host, n, b, xcds, slots, counted):
     out = band_host("pair", n, b, xcds, slots, counted)
     assert out.count("ended") == 6
+
+
+# (equations, half-bandwidth): one to five tile rows, a ragged last block, full
+# bands in one, two and three blocks, helpers
+@pytest.mark.parametrize("n,b", [(40, 10), (128, 127), (300, 40), (310, 309), (330, 300), (400, 150), (600, 599), (1300, 600)])
+def test_schedules_and_sweeps_agree(band_host, n, b):
+    assert band_host("solve", n, b).count("backward error") == 6

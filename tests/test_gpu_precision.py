@@ -87,8 +87,8 @@ def test_fp32_precision_mode_panel_msal_path(n, steps, refine):
 
 @pytest.mark.parametrize("sweeps", [1, 2])
 def test_fp32_precision_mode_under_every_sweep_schedule(sweeps):
-    """The FP32 band's solves on the two-product row step and on the
-    look-ahead system (both sweeps coupled two rows back) against the chain
+    """The FP32 band's solves on the two-product row step and in blocks of
+    four tile rows against the chain
     matrices: the same converged steps, the displacements to 1e-5 (the bar of
     the FP32 paths above; the schedules differ only in rounding)."""
     path = panel(8)

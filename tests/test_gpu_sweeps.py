@@ -5,9 +5,8 @@ both give a normwise backward error at the FP64 round-off level for random
 right-hand sides, on models whose band shapes cover the kernels' edge cases --
 a single tile row (nt = 1), odd and even numbers of tile rows, and 1, 2 and
 more tiles below the diagonal -- and the arc-length paths of both schedules
-agree with the oracle.  The look-ahead systems (CB_SWEEP_LOOK2, rows coupled
-two and more back, and CB_SWEEP_LOOK3, three and more back) are held to the
-same bars."""
+agree with the oracle.  The block sweeps (CB_SWEEP_LOOK2, and CB_SWEEP_LOOK3,
+another name for it) are held to the same bars."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
