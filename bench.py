@@ -99,13 +99,15 @@ def kernel_model(info, sweeps: str = "chain") -> dict:
     }
 
 
-# HBM bytes per launch of the batch's factor kernel on the default workload,
-# from two rocprofv3 counter runs (FETCH_SIZE, then WRITE_SIZE, KiB per
-# dispatch), scaled by what the same counters read for an elementwise copy of
-# 256 MiB (FETCH_SIZE x 2.000, WRITE_SIZE x 1.000): k_band_factor_models over
-# the 13 rounds of 5 time steps of the 512 frames.
+# HBM bytes of the dominant kernels on the default workloads, from two rocprofv3
+# counter runs each (FETCH_SIZE, then WRITE_SIZE, KiB per dispatch), scaled by
+# what the same counters read for an elementwise copy of 256 MiB (FETCH_SIZE x
+# 2.000, WRITE_SIZE x 1.000): k_band_factor over the 256x256 panel's
+# factorization, per tile column (6168 of them), k_band_factor_models per launch
+# over 66 launches of a run of 5 time steps of the 512 frames.
 MEASURED_TRAFFIC = {
-    "band_factor_models": (1679014.64 * 2.0 + 3575412.50) * 1024.0,
+    "band_column": (37554753.62 * 2.0 + 10582052.03) * 1024.0 / 6168,
+    "band_factor_models": (1465778.71 * 2.0 + 3421711.34) * 1024.0,
 }
 TRAFFIC_SOURCE = ("rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE runs, KiB per dispatch scaled by a 256 MiB "
                   "copy (x2.000, x1.000)")
@@ -127,7 +129,7 @@ def roofline(info, ktimes: dict, default_workload: bool, sky: dict | None = None
     bound, work, unit = kernel_model(info, sweeps)[name]
     nt = (info.neq + TILE - 1) // TILE
     if sky is not None and name == "band_column":
-        work = sky["factor_flops"] / nt          # a factorization is nt column launches
+        work = sky["factor_flops"] / nt          # a factorization is nt tile columns
     elif sky is not None and name in ("band_fwd_sweep", "band_bwd_sweep"):
         work = sky["sweep_bytes"]
     avg_s = ms / 1000.0 / max(launches, 1)
@@ -140,9 +142,9 @@ def roofline(info, ktimes: dict, default_workload: bool, sky: dict | None = None
            "frac": achieved / peak, "traffic": traffic, "avg_launch_us": 1e6 * avg_s, "launches": launches,
            "share_of_kernel_time": ms / sum(v[0] for v in ktimes.values())}
     if sky is not None and name == "band_column":
-        out["work_basis"] = "sum(kht^2) flops of the skyline factorization / nt launches"
+        out["work_basis"] = "sum(kht^2) flops of the skyline factorization / nt tile columns"
     if traffic is not None:
-        out["traffic_unit"] = "B per launch"
+        out["traffic_unit"] = "B per tile column" if name == "band_column" else "B per launch"
         out["traffic_source"] = TRAFFIC_SOURCE
     if sky is not None:
         # the two sweeps of every solve: algorithmic bytes (the skyline factor

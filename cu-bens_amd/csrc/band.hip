@@ -734,21 +734,23 @@ __global__ void __launch_bounds__(NTH) k_tile_update(R* __restrict__ tiles, cons
 //   corner(I)  (I, I) likewise, with P_{I,I-2}
 // One column's critical path is then the chain's own P, U, D or half the loop
 // Linv_{J-2} -> near(J) -> chain -> Linv_J, whichever is longer.  The chain is:
-// 17.9 us a column (200 x 200 panel, 12.1 of it the diagonal task), against
+// 17.6 us a column (256 x 256 panel, 12.1 of it the diagonal task), against
 // 21.2 us for a launch per column whose workgroups loaded and stored every
 // tile they updated.  The other workgroups of a band of 25 tiles need about 3 us
-// a column of the whole chip's matrix units, so they keep up.  Counters (zero
+// a column of the whole chip's matrix units, so they keep up; from about 31 tiles
+// on the updates' reads of two tiles each set the pace, 20.2 us a column with 38
+// tiles, 32 with 98 and 134 with 219 (a launch per column: 33, 56 and 264).
+// Counters (zero
 // before the launch): P_ROW the columns of a tile row that its tile() tasks have
 // finished, P_LAST L_{J,J-1} stored, P_DIAG D_J and Linv_J stored, P_NEAR and
 // P_NEAR2 a row's two last tiles handed over, P_PART tile (I, I-2) handed over (in
 // slot (I, I) of tiles, which holds nothing else).
 // Workgroups take their tasks as they start (start_number) and wait only on
-// earlier tasks and on the chain.  The chain, the first task,
-// waits on near and corner of the column it has reached, whose own waits are
-// on earlier columns, so the earliest unfinished task beside it can always go
-// on; every wait ends as long as there is room beside the chains, which keep a
-// CU each for a whole factorization.  Waits are
-// bounded anyway.  Order: the chain, then by column J = 0, 1, ..: tile(J+2, J),
+// earlier tasks and on the chain.  The chain, the first task, waits on near and
+// corner of the column it has reached, whose own waits are on earlier columns,
+// so the earliest unfinished task beside it can always go on; every wait ends
+// as long as there is room beside the chains, which keep a CU each for a whole
+// factorization.  Waits are bounded anyway.  Order: the chain, then by column J = 0, 1, ..: tile(J+2, J),
 // near(J+2), corner(J+2), tile(J+3, J) .. tile(J+m, J), m = min(w, nt-1-J)
 // (m + 1 workgroups, none for m < 2).
 // The band is assembled in tiles_t and the factor goes to tiles: no line of
@@ -1545,8 +1547,8 @@ __global__ void __launch_bounds__(256) k_bwd_sweep_m(const R* __restrict__ tiles
 // time the front takes to pass it.  A block has 4 (gh + 1) workgroups of 512
 // threads: for each row gh helpers, each with up to HT tiles of the older
 // rows, which leave partial sums, and one that finishes the row.
-// 256 x 256 panel (6168 rows, 25 tiles below the diagonal): 2.44 / 2.50 ms
-// forward / backward (2.5 TB/s of 6.0 GB) and 2.7 ms to form the matrices per
+// 256 x 256 panel (6168 rows, 25 tiles below the diagonal): 2.46 / 2.44 ms
+// forward / backward (2.2 TB/s of 5.3 GB) and 2.7 ms to form the matrices per
 // factorization; one row at a time took 6.2 / 6.5 ms, and systems that
 // decoupled each row from the one or two before 5.1 / 5.2 ms with 11 ms of
 // forming.  A band of a single block has nothing to overlap and takes the
